@@ -65,6 +65,9 @@ _SIGNATURES = {
                                    _L, _P], _I),
     "gdn_chunk_prefill_generic": ([_P, _L, _P, _L, _P, _L, _P, _P, _I, _P, _P, _P, _I, _P, _L, _P, _I, _I, _I,
                                    _I, _I, _I, _I, _I, _P], _I),
+    "gdn_chunk_prefill_generic_workspace_bytes": ([_I, _I, _I, _I, _I], _L),
+    "gdn_chunk_prefill_generic_ws": ([_P, _L, _P, _L, _P, _L, _P, _P, _I, _P, _P, _P, _I, _P, _L, _P, _I, _I, _I,
+                                      _I, _I, _I, _I, _I, _P, _L, _P], _I),
 }
 
 _lib = None

@@ -181,9 +181,8 @@ def chunk_gated_delta_rule(query, key, value, g, beta, chunk_size=64, initial_st
     dev = query.device
     if fast:
         cu, seq_chunk0, nseq, seq_len, total_chunks = _chunk_table(B, T, cu_seqlens, dev)
-    else:  # the generic kernel walks each sequence itself: no chunk table
-        cu, nseq, seq_len = _seq_args(B, T, cu_seqlens, dev)
-        seq_chunk0, total_chunks = None, 0
+    else:  # the generic kernels number chunks by sequence: no chunk table, but the lengths' bound
+        cu, _, nseq, seq_len, _ = _chunk_table(B, T, cu_seqlens, dev)
     q, qs = _tokens_view(query, "query")
     k, ks = _tokens_view(key, "key")
     v, vs = _tokens_view(value, "value")
@@ -212,10 +211,12 @@ def chunk_gated_delta_rule(query, key, value, g, beta, chunk_size=64, initial_st
         final = torch.empty(nseq, Hv, D, Dv, dtype=torch.float32, device=dev) if output_final_state else None
     out = torch.empty(B, T, Hv, Dv, dtype=query.dtype, device=dev)
     if not fast:
-        _lib.call("gdn_chunk_prefill_generic", _lib.ptr(q), qs, _lib.ptr(k), ks, _lib.ptr(v), vs, _lib.ptr(g32),
+        wbytes = int(_lib.lib().gdn_chunk_prefill_generic_workspace_bytes(nseq, seq_len, Hv, D, Dv))
+        work = torch.empty(max(wbytes, 1), dtype=torch.uint8, device=dev)
+        _lib.call("gdn_chunk_prefill_generic_ws", _lib.ptr(q), qs, _lib.ptr(k), ks, _lib.ptr(v), vs, _lib.ptr(g32),
                   _lib.ptr(beta), _lib.dtype_code(beta), _lib.ptr(init), _lib.ptr(final), _lib.ptr(rows), n_rows,
                   _lib.ptr(out), B * T, _lib.ptr(cu), nseq, seq_len, Hqk, Hv, D, Dv, _lib.dtype_code(query),
-                  int(bool(use_qk_l2norm_in_kernel)), _lib.stream_of(query))
+                  int(bool(use_qk_l2norm_in_kernel)), _lib.ptr(work), wbytes, _lib.stream_of(query))
         return out, final
     wbytes = int(_lib.lib().gdn_chunk_prefill_workspace_bytes(total_chunks, nseq, Hv))
     work = torch.empty(max(wbytes, 1), dtype=torch.uint8, device=dev)

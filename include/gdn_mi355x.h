@@ -153,6 +153,25 @@ int gdn_chunk_prefill_generic(const void* q, int64_t q_stride, const void* k, in
                               int Dv, int in_dtype, int use_qk_l2norm, void* stream);
 
 /*
+ * gdn_chunk_prefill_generic with a workspace: the same rule, in fp32 throughout, in two kernels -- the
+ * state-independent part of every chunk in parallel, then the state chain over 16 value columns per
+ * workgroup.  Arguments as gdn_chunk_prefill_generic, except that with cu_seqlens seq_len must be an
+ * upper bound of every sequence's length (a bound below a sequence's true length drops that
+ * sequence's later chunks), and out must be 16-byte aligned.
+ *   workspace: 16-byte aligned, gdn_chunk_prefill_generic_workspace_bytes(nseq, seq_len, Hv, Dk, Dv)
+ *     bytes (-1 for bad sizes): about (3 Dk + Dv + 40) * 256 bytes per (chunk, value head), capped near
+ *     256 MiB (longer calls run in windows of chunks, several launches each); contents are scratch.
+ */
+int64_t gdn_chunk_prefill_generic_workspace_bytes(int nseq, int max_len, int Hv, int Dk, int Dv);
+int gdn_chunk_prefill_generic_ws(const void* q, int64_t q_stride, const void* k, int64_t k_stride,
+                                 const void* v, int64_t v_stride, const float* g, const void* beta,
+                                 int beta_dtype, const float* initial_state, float* final_state,
+                                 const int32_t* state_rows, int n_rows, void* out, int64_t total_tokens,
+                                 const int32_t* cu_seqlens, int nseq, int seq_len, int Hqk, int Hv, int Dk,
+                                 int Dv, int in_dtype, int use_qk_l2norm, void* workspace,
+                                 int64_t workspace_bytes, void* stream);
+
+/*
  * Bytes of device workspace gdn_chunk_prefill needs for `total_chunks` 64-token chunks of `nseq`
  * sequences and Hv value heads (-1 for bad sizes): the segment table and flags (a few bytes per
  * sequence and per segment), the fp32 transition maps of the segments that have a successor (at

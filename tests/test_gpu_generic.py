@@ -187,3 +187,48 @@ def test_generic_sweep(gdn, oracle, dev, i):
     otol, stol = (FP32_TOL, FP32_TOL) if dtype == torch.float32 else (1e-2, 1e-3)
     assert rel_l2(o.float(), o_ref.float()) <= otol, rel_l2(o.float(), o_ref.float())
     assert rel_l2(s, s_ref) <= stol, rel_l2(s, s_ref)
+
+
+@pytest.mark.parametrize("dtype,Dk,Dv,aligned", [
+    (torch.float32, 64, 64, True),    # groups of sequences (the workspace cap holds 221 here) and windows of chunks
+    (torch.float16, 16, 128, False),  # two value slices, token strides that rule out the vector loads
+])
+def test_generic_windows_and_groups_match_the_workspace_free_kernel(gdn, oracle, dev, dtype, Dk, Dv, aligned):
+    """230 packed sequences of 0, 1, 63, 64, 65 and 130 tokens, states in and out: the two-kernel form against the
+    one-kernel form on every value (fp32 sums in another order over at most 128 terms a product and 3 chunks: 1e-5,
+    rounded once to a 16-bit output: 2^-10), and against the oracle on one sequence of each length."""
+    from importlib import import_module
+    lib = import_module(gdn.__name__ + "._lib")
+    Hk, Hv, lens = 8, 16, [(0, 1, 63, 64, 65, 130)[i % 6] for i in range(230)]
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    T, r = cu[-1], torch.Generator().manual_seed(91)
+    pad = 0 if aligned else 3
+    wide = lambda H, d: torch.randn(1, T, H * d + pad, generator=r).to(dtype)
+    q, k, v = (x[..., :H * d].reshape(1, T, H, d) if not pad else x[..., :H * d].unflatten(-1, (H, d))
+               for x, H, d in ((wide(Hk, Dk), Hk, Dk), (wide(Hk, Dk), Hk, Dk), (wide(Hv, Dv), Hv, Dv)))
+    beta, g = torch.sigmoid(torch.randn(1, T, Hv, generator=r)), -0.1 * torch.rand(1, T, Hv, generator=r)
+    s0 = 0.1 * torch.randn(len(lens), Hv, Dk, Dv, generator=r)
+    qd, kd, vd, gd, bd, sd = _dev(dev, q, k, v, g, beta, s0)
+    if pad:  # .to() packs: rebuild the padded token stride on the device
+        qd, kd, vd = (torch.nn.functional.pad(x.flatten(2), (0, pad))[..., :x.shape[2] * x.shape[3]]
+                      .unflatten(-1, x.shape[2:]) for x in (qd, kd, vd))
+        assert qd.stride(1) % 4
+    o, s = gdn.chunk_gated_delta_rule(qd, kd, vd, gd, bd, initial_state=sd, output_final_state=True,
+                                      use_qk_l2norm_in_kernel=True, cu_seqlens=cu)
+    table = gdn.Varlen(cu, T, dev)
+    o1, s1 = torch.empty_like(o), torch.empty_like(s)
+    p = lib.ptr
+    lib.call("gdn_chunk_prefill_generic", p(qd), qd.stride(1), p(kd), kd.stride(1), p(vd), vd.stride(1), p(gd), p(bd),
+             lib.dtype_code(bd), p(sd), p(s1), None, len(lens), p(o1), T, p(table.cu), len(lens), 0, Hk, Hv, Dk, Dv,
+             lib.dtype_code(qd), 1, lib.stream_of(qd))
+    torch.cuda.synchronize()
+    assert rel_l2(o, o1) <= (1e-5 if dtype == torch.float32 else 2.0 ** -10) and rel_l2(s, s1) <= 1e-5
+    for i in (0, 1, 2, 3, 4, 5, 222, 223, 227, 229):  # both groups
+        sl = slice(cu[i], cu[i + 1])
+        o_ref, s_ref = oracle.chunk_gated_delta_rule_v2(q[:, sl].repeat_interleave(2, 2), k[:, sl].repeat_interleave(2, 2),
+                                                        v[:, sl], g[:, sl], beta[:, sl], 64, s0[i:i + 1], True, True)
+        assert rel_l2(s[i], s_ref[0]) <= (FP32_TOL if dtype == torch.float32 else 1e-3)
+        if lens[i]:
+            assert rel_l2(o[:, sl].float(), o_ref.float()) <= (FP32_TOL if dtype == torch.float32 else 1e-2)
