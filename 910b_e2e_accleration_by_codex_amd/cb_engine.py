@@ -309,7 +309,7 @@ def gqa_decode_attention(proj, pos, q_norm, k_norm, inv_freq, k_cache_t, v_cache
     positions 0..pos, times sigmoid(gate).  proj [N, (2 nh + 2 kv) hd] bf16 (per head q then gate, then
     k, then v), or that projection's Partials (decode_linear_partial: reduced here, no reduction
     launch), pos [N] int64 on the device.  Returns the gated output [N, nh * hd] bf16 (o_proj's
-    input).  Three HIP launches, capturable in a graph."""
+    input).  Two HIP launches (three from Partials), capturable in a graph."""
     nh, kv, hd = n_heads, kv_heads, head_dim
     part = proj if isinstance(proj, Partials) else None
     if part is not None:

@@ -421,7 +421,7 @@ int gdn_swiglu_partial(const float* part, int splits, void* out, int M, int64_t 
  * slots.  It has no counterpart inside the reference's GDN path: it is the attention layer the
  * reference's engine runs between its GDN layers, HF Qwen3_5Attention.forward
  * (transformers modeling_qwen3_5.py:629-700: gated q, q/k Qwen3_5RMSNorm, partial rotary,
- * softmax(q k^T / sqrt(hd)) v, times sigmoid(gate)), here in three launches on a per-slot cache.
+ * softmax(q k^T / sqrt(hd)) v, times sigmoid(gate)), here in two launches on a per-slot cache.
  *   proj [N, proj_stride] bf16: per query head h its q (hd) then its gate (hd) at h * 2hd, then the
  *     kv key rows (hd each) at 2 nh hd, then the kv value rows at (2 nh + kv) hd.
  *   pos [N] int64 (device): the position of the new token; it is written to the caches there and
@@ -442,7 +442,8 @@ int gdn_attn_decode(const void* proj, int64_t proj_stride, const int64_t* pos, c
                     float eps, void* stream);
 /* The same with the projection given as its split-K partial sums (gdn_decode_linear_packed_partial):
  * part [splits][N][(2 nh + 2 kv) hd] fp32; every value is bf16(sum over splits, in split order), as in
- * the reduced projection, so the result is identical and the reduction launch disappears. */
+ * the reduced projection, so the result is identical; a launch of its own reduces and prepares the q, k and
+ * v rows, in place of the reduction. */
 int gdn_attn_decode_partial(const float* part, int splits, const int64_t* pos, const void* q_norm_w,
                             const void* k_norm_w, const float* inv_freq, void* k_cache_t, void* v_cache, void* out,
                             int64_t out_stride, float* work, int64_t work_bytes, int N, int nh, int kv, int hd, int rd,

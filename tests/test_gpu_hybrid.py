@@ -169,6 +169,38 @@ def test_gqa_decode_attention_vs_fp32(gdn, dev, nh, kv, hd, pos, T):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("nh,kv,hd,T", [
+    (6, 1, 256, 516), (16, 2, 256, 576),  # 8 waves a split; rows that do and do not fill whole cache lines
+    (8, 2, 128, 516), (4, 4, 64, 516),    # 4 waves a split
+])
+def test_gqa_decode_attention_wave_and_split_edges(gdn, dev, nh, kv, hd, T):
+    """Positions at the edges of a lane's 4 tokens, a wave's 64 and a split's 256, with NaN in every cache
+    entry past each slot's position (and at it: the new token replaces what was there): the outputs match
+    the fp32 loop and hold no NaN.  A position past the cache writes nothing and attends to all of it."""
+    from importlib import import_module
+    cb = import_module(PKG_NAME + ".cb_engine")
+    pos = [0, 3, 4, 63, 64, 127, 128, 255, 256, 319, T - 1, T + 3]
+    N, rd, eps = len(pos), hd // 4, 1e-6
+    g_ = torch.Generator().manual_seed(hd + nh + T)
+    bf = torch.bfloat16
+    proj = torch.randn(N, (2 * nh + 2 * kv) * hd, generator=g_).to(bf)
+    qn, kn = (0.1 * torch.randn(hd, generator=g_)).to(bf), (0.1 * torch.randn(hd, generator=g_)).to(bf)
+    inv = 1.0 / (10000.0 ** (torch.arange(0, rd, 2).float() / rd))
+    kt = torch.randn(N, kv, hd, T, generator=g_).to(bf)
+    vc = torch.randn(N, kv, T, hd, generator=g_).to(bf)
+    for n, p in enumerate(pos):
+        kt[n, :, :, p:], vc[n, :, p:] = float("nan"), float("nan")
+    kt_d, vc_d = kt.to(dev), vc.to(dev)
+    out = cb.gqa_decode_attention(proj.to(dev), torch.tensor(pos, device=dev), qn.to(dev), kn.to(dev), inv.to(dev), kt_d,
+                                  vc_d, nh, kv, hd, rd, eps).cpu().float()
+    assert not out.isnan().any()
+    assert torch.equal(kt_d[-1].cpu(), kt[-1]) and torch.equal(vc_d[-1].cpu(), vc[-1])
+    ref = _attn_reference(proj[:-1], torch.tensor(pos[:-1]), qn, kn, inv, kt[:-1], vc[:-1], nh, kv, hd, rd, eps)
+    for n in range(N - 1):  # bf16 probabilities and output: 2^-9 a value
+        assert rel_l2(out[n], ref[n]) <= OUT_TOL, pos[n]
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("nh,kv,hd,H", [(4, 2, 64, 512), (24, 4, 256, 5120)])
 def test_gqa_decode_attention_from_partials(gdn, dev, nh, kv, hd, H):
     """The attention fed the q|gate|k|v projection's split-K partials gives exactly what it gives on the
