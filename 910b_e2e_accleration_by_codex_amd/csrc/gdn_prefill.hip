@@ -286,6 +286,7 @@ struct SegTable {
   const int32_t* seg0;
   const int32_t* order;  // output pass: segments longest first (nullptr: in index order)
   int nseq, seq_len, L;
+  int walk;  // pairs without warm-ups walk their whole sequence in one workgroup (no summary pass): walk_pays()
   __device__ __forceinline__ int nch(int s) const {
     return cu ? chunk0[s + 1] - chunk0[s] : (seq_len + pf::CH - 1) / pf::CH;
   }
@@ -1326,14 +1327,19 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
     mode = (item & 1) ? kSegA : kSegB;
     if (seq_warm_ok(tab, warm, Hv, h, s)) return;  // the output pass warms up instead
   }
-  const bool warm_path = kPass == 0 && slot >= 0 && seq_warm_ok(tab, warm, Hv, h, s);
+  const int nch_s = tab.nch(s), nseg_s = tab.nseg_of(nch_s);
+  const bool warm_ok = kPass == 0 && nseg_s > 1 && (slot >= 0 || tab.walk) && seq_warm_ok(tab, warm, Hv, h, s);
+  // a pair without warm-ups, short sequences: segment 0's workgroup runs all of it
+  const bool walk = kPass == 0 && tab.walk && nseg_s > 1 && !warm_ok;
+  if (walk && idx > 0) return;
+  const bool warm_path = slot >= 0 && warm_ok;
   // the output pass of a later segment on the exact path forms its initial state from the summaries of
   // the idx slots before it (ts_first .. ts_first + idx - 1)
   const int combine_steps = (kPass == 0 && slot >= 0 && !warm_path) ? idx : 0;
   const int ts_first = tab.first_slot(s);
   const int kh = h / (Hv / Hqk);
-  const int nch_s = tab.nch(s), c_begin = idx * tab.L;
-  const int n = nch_s - c_begin < tab.L ? nch_s - c_begin : tab.L;
+  const int c_begin = idx * tab.L;
+  const int n = walk || nch_s - c_begin < tab.L ? nch_s - c_begin : tab.L;
   const int64_t t_seq = tab.start(s);
   const int Ls = tab.len(s);
   float* tslot = slot >= 0 ? trans + ((int64_t)slot * Hv + h) * sg::kTrans : nullptr;
@@ -1628,7 +1634,7 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
     }
     // the state after the segment
     if (mode == kSegOut) {
-      if (final_state && idx == tab.nseg_of(nch_s) - 1) {
+      if (final_state && (walk || idx == nseg_s - 1)) {
         const int r0 = state_row(rows, n_rows, s);
         if (r0 >= 0) {
           float* dst = final_state + ((int64_t)r0 * Hv + h) * D * D;
@@ -2042,6 +2048,19 @@ SegLayout seg_layout(int64_t total_chunks, int nseq, int Hv) {
   l.bytes = l.off_knorm + total_chunks * Hv * (int64_t)(kr::FLOATS * 4);
   return l;
 }
+// Whether (sequence, value head) pairs without warm-ups walk their whole sequence in one workgroup instead
+// of taking the exact path; the call then needs no summary launch (2-3 us when every pair warms up).
+// In chunk steps of the walk (4.8 us each), the exact path costs about L for the outputs, 1.35 L per round
+// of 256 summary workgroups, and 0.75 per segment to combine: fitted on whole calls of 130 to 3000
+// tokens at 16, 32 and 48 value heads, e.g. slow decay, exact path against walk: 353 tokens x 48 heads
+// 54 / 48 us, 517 x 48 69 / 63, 700 x 48 78 / 73, 1000 x 48 93 / 97, 517 x 32 57 / 62, 517 x 16 54 / 60.
+// With the fused norm a step with outputs takes a third longer, the summaries' steps do not (the layer at
+// 517 tokens x 48 heads: 83.4 us on the exact path, 85.7 walked).
+bool walk_pays(int64_t max_seq_chunks, const SegLayout& lay, int Hv, bool norm) {
+  const int64_t segs = (max_seq_chunks + lay.L - 1) / lay.L, rounds = (2 * lay.nslots * Hv + 255) / 256;
+  const int64_t more = (27 * rounds * lay.L + 15 * (segs - 1)) * (norm ? 3 : 4) / 4;
+  return segs > 1 && 20 * max_seq_chunks <= 20 * lay.L + more;
+}
 }  // namespace
 
 extern "C" int64_t gdn_chunk_prefill_workspace_bytes(int64_t total_chunks, int nseq, int Hv) {
@@ -2109,8 +2128,12 @@ int chunk_prefill_impl(const void* q, int64_t q_stride, const void* k, int64_t k
     int rc = check_launch("gdn_chunk_prefill(table)");
     if (rc) return rc;
   }
+  // A sequence spans several segments only beyond L chunks: seq_len is the uniform length, or for
+  // packed sequences an upper bound of the longest one (0: unknown)
+  const int64_t max_seq_chunks = seq_len > 0 ? ((int64_t)seq_len + pf::CH - 1) / pf::CH : total_chunks;
+  const int walk = walk_pays(max_seq_chunks, lay, Hv, norm_mode != 0) ? 1 : 0;
   const SegTable tab{cu_seqlens, seq_chunk0, cu_seqlens ? seg0 : nullptr, cu_seqlens ? order : nullptr, nseq, seq_len,
-                     (int)lay.L};
+                     (int)lay.L, walk};
   if (total_chunks > 0) {  // the intra-chunk inverses, one wave per (chunk, value head)
     const int64_t items = total_chunks * Hv;
     const unsigned gi = (unsigned)((items + 3) / 4);
@@ -2138,10 +2161,7 @@ int chunk_prefill_impl(const void* q, int64_t q_stride, const void* k, int64_t k
     else GDN_SEG_LAUNCH(float);
 #undef GDN_SEG_LAUNCH
   };
-  // A sequence spans several segments only beyond L chunks: seq_len is the uniform length, or for
-  // packed sequences an upper bound of the longest one (0: unknown)
-  const int64_t max_seq_chunks = seq_len > 0 ? ((int64_t)seq_len + pf::CH - 1) / pf::CH : total_chunks;
-  if (lay.nslots > 0 && max_seq_chunks > lay.L) {  // segment summaries and their combination where no warm-up fits
+  if (!walk && lay.nslots > 0 && max_seq_chunks > lay.L) {  // segment summaries and their combination where no warm-up fits
     launch(1, lay.nslots * Hv * 2);
     int rc = check_launch("gdn_chunk_prefill(summary)");
     if (rc) return rc;
@@ -2288,7 +2308,7 @@ extern "C" int gdn_chunk_prefill_inverse(const void* k, int64_t k_stride, const 
     const int rc = check_launch("gdn_chunk_prefill_inverse(table)");
     if (rc) return rc;
   }
-  const SegTable tab{cu_seqlens, seq_chunk0, cu_seqlens ? seg0 : nullptr, nullptr, nseq, seq_len, (int)lay.L};
+  const SegTable tab{cu_seqlens, seq_chunk0, cu_seqlens ? seg0 : nullptr, nullptr, nseq, seq_len, (int)lay.L, 0};
   uint8_t* tfrag = work + lay.off_tfrag;
   float* knorm = (float*)(work + lay.off_knorm);
   int* warm = (int*)(work + lay.off_warm);

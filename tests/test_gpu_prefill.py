@@ -464,3 +464,34 @@ def test_gating(gdn, oracle, dev):
     assert torch.equal(beta.cpu(), beta_ref)
     assert rel_l2(g, g_ref) <= 1e-6
 
+
+
+@pytest.mark.parametrize("lens,n_rows", [([384], 1), ([385], 1), ([100, 0, 384, 65, 1], 7), ([700, 64, 353], 3)])
+def test_chunk_prefill_short_sequences_walk(gdn, oracle, dev, lens, n_rows):
+    """Short sequences: heads without a warm-up are walked from the start by their first segment's workgroup (384
+    tokens, 6 chunks, at these sizes; 385 tokens already take the summaries, as 700 do), while the other heads of
+    the call warm up.  Initial and final states in slot rows, in place; every (sequence, head) against the oracle."""
+    Hk, Hv, T = 2, 4, sum(lens)
+    q, k, v, g, beta, _ = _gdn_inputs(T, Hk, Hv, seed=T, state=False)
+    g[..., 0] *= 10.0
+    g[..., 1] *= 0.01
+    g[..., 2] = 0.0
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    slots = 0.02 * torch.randn(n_rows, Hv, 128, 128, generator=torch.Generator().manual_seed(5))
+    rows = list(range(n_rows))[::-1][:len(lens)]
+    o_ref, s_ref = oracle.chunk_gated_delta_rule_varlen(_rep(q, 2), _rep(k, 2), v, g, beta, torch.tensor(cu), 64,
+                                                        slots[rows], True, True)
+    sd = slots.to(dev)
+    o, _ = gdn.chunk_gated_delta_rule(q.to(dev), k.to(dev), v.to(dev), g.to(dev), beta.to(dev), initial_state=sd,
+                                      cu_seqlens=cu, state_rows=rows, final_state_out=sd,
+                                      use_qk_l2norm_in_kernel=True)
+    for i in range(len(lens)):
+        for h in range(Hv):
+            if lens[i]:
+                sl = slice(cu[i], cu[i + 1])
+                assert rel_l2(o[:, sl, h], o_ref[:, sl, h]) <= OUT_TOL, (i, h)
+            assert rel_l2(sd[rows[i], h], s_ref[i, h]) <= STATE_TOL, (i, h)
+    for spare in set(range(n_rows)) - set(rows):
+        assert torch.equal(sd[spare].cpu(), slots[spare])
