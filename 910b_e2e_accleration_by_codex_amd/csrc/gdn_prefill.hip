@@ -484,6 +484,41 @@ __device__ __forceinline__ int64_t xcd_range_item(int64_t b, int64_t n) {
   return b >= 8 * per ? b : (b % 8) * per + b / 8;
 }
 
+// The decode conv state each sequence leaves: its last K inputs, the front filled from its history
+// row (or zeros) when the sequence is shorter than K -- an empty sequence keeps its history.  One
+// thread per (sequence, channel) reads its old row entries before writing them, so `history` and
+// `state` may be the same slot rows.
+__device__ __forceinline__ void capture_one(int64_t i, const uint16_t* __restrict__ x, int64_t x_stride,
+                                            const uint16_t* history, const int32_t* __restrict__ hist_rows,
+                                            uint16_t* state, const int32_t* __restrict__ state_rows, int n_rows,
+                                            const int32_t* __restrict__ cu, int nseq, int seq_len, int C, int K) {
+  if (i >= (int64_t)nseq * C) return;
+  const int s = (int)(i / C), c = (int)(i % C);
+  const int orow = state_row(state_rows, n_rows, s);
+  if (orow < 0) return;
+  const int hrow = history ? state_row(hist_rows, n_rows, s) : -1;
+  const int64_t s_lo = cu ? (int64_t)cu[s] : (int64_t)s * seq_len;
+  const int64_t L = cu ? (int64_t)cu[s + 1] - s_lo : seq_len;
+  uint16_t win[8];
+  for (int j = 0; j < K; ++j) {  // win[j] = input K - j before the end of the sequence
+    const int64_t tok = L - K + j;  // position inside the sequence
+    if (tok >= 0) win[j] = x[(s_lo + tok) * x_stride + c];
+    else win[j] = hrow >= 0 ? history[((int64_t)hrow * C + c) * K + (K + tok)] : (uint16_t)0;
+  }
+  for (int j = 0; j < K; ++j) state[((int64_t)orow * C + c) * K + j] = win[j];
+}
+// The capture as further workgroups of the inverse kernel's grid (blocks 0 .. n - 1, the launch after the
+// conv's): for a prompt continuing in its slot, whose history rows, which the conv reads, are the state rows.
+// A launch of its own took 4.8 us.
+struct CaptureArgs {
+  int n;  // workgroups (a multiple of 8, so the items keep their XCDs; 0: no capture)
+  const uint16_t* x;
+  int64_t x_stride;
+  uint16_t* rows_buf;  // history and state
+  const int32_t* rows;
+  int n_rows, C, K;
+};
+
 // One wave per (chunk, value head) item (item = chunk slot * Hv + value head; a workgroup's 4 waves
 // are independent, so a wave past the end simply exits).  Lane (i, g) holds K[16 t + i][32 s + 8 g
 // .. + 7] for token tiles t and k-blocks s < 4: the A fragment of tile t and, as K^T, the B
@@ -497,15 +532,20 @@ __global__ __launch_bounds__(pf::NT, 2) void inv_kernel(const uint16_t* __restri
                                                        const int32_t* __restrict__ seq_chunk0, int nseq, int seq_len,
                                                        int64_t items, int Hqk, int Hv, int use_l2,
                                                        uint8_t* __restrict__ tfrag, float* __restrict__ knorm,
-                                                       SegTable tab, int* __restrict__ warm) {
+                                                       SegTable tab, int* __restrict__ warm, CaptureArgs cap) {
   using namespace pf;
+  if ((int)blockIdx.x < cap.n) {
+    capture_one((int64_t)blockIdx.x * NT + threadIdx.x, cap.x, cap.x_stride, cap.rows_buf, cap.rows, cap.rows_buf,
+                cap.rows, cap.n_rows, cu, nseq, seq_len, cap.C, cap.K);
+    return;
+  }
   __shared__ float sdec[4][2][CH];                // per wave: G and beta by token
   __shared__ float strp[4][4 * 16 * kTrPitch];    // per wave: 4 transpose tiles
   const int t = threadIdx.x, lane = t & 63, c16 = lane & 15, g4 = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);  // the item is wave-uniform: scalar control flow
   // the 8 workgroups of one chunk's 32 value heads share an XCD, so the chunk's g and beta lines
   // (one token's heads per line) come from HBM once per chunk, not once per XCD
-  const int64_t item = xcd_range_item(blockIdx.x, gridDim.x) * 4 + w;
+  const int64_t item = xcd_range_item(blockIdx.x - cap.n, gridDim.x - cap.n) * 4 + w;
   if (item >= items) return;
   const int slot = (int)(item / Hv), h = (int)(item % Hv);
   const int r = Hv / Hqk, hk = h / r;
@@ -1841,29 +1881,6 @@ __global__ __launch_bounds__(256) void conv_prefill_kernel(const uint16_t* __res
               total_tokens, cu, nseq, seq_len, C);
 }
 
-// The decode conv state each sequence leaves: its last K inputs, the front filled from its history
-// row (or zeros) when the sequence is shorter than K -- an empty sequence keeps its history.  One
-// thread per (sequence, channel) reads its old row entries before writing them, so `history` and
-// `state` may be the same slot rows.
-__device__ __forceinline__ void capture_one(int64_t i, const uint16_t* __restrict__ x, int64_t x_stride,
-                                            const uint16_t* history, const int32_t* __restrict__ hist_rows,
-                                            uint16_t* state, const int32_t* __restrict__ state_rows, int n_rows,
-                                            const int32_t* __restrict__ cu, int nseq, int seq_len, int C, int K) {
-  if (i >= (int64_t)nseq * C) return;
-  const int s = (int)(i / C), c = (int)(i % C);
-  const int orow = state_row(state_rows, n_rows, s);
-  if (orow < 0) return;
-  const int hrow = history ? state_row(hist_rows, n_rows, s) : -1;
-  const int64_t s_lo = cu ? (int64_t)cu[s] : (int64_t)s * seq_len;
-  const int64_t L = cu ? (int64_t)cu[s + 1] - s_lo : seq_len;
-  uint16_t win[8];
-  for (int j = 0; j < K; ++j) {  // win[j] = input K - j before the end of the sequence
-    const int64_t tok = L - K + j;  // position inside the sequence
-    if (tok >= 0) win[j] = x[(s_lo + tok) * x_stride + c];
-    else win[j] = hrow >= 0 ? history[((int64_t)hrow * C + c) * K + (K + tok)] : (uint16_t)0;
-  }
-  for (int j = 0; j < K; ++j) state[((int64_t)orow * C + c) * K + j] = win[j];
-}
 __global__ void conv_state_capture_kernel(const uint16_t* __restrict__ x, int64_t x_stride,
                                           const uint16_t* history, const int32_t* __restrict__ hist_rows,
                                           uint16_t* state, const int32_t* __restrict__ state_rows, int n_rows,
@@ -2076,7 +2093,7 @@ int chunk_prefill_impl(const void* q, int64_t q_stride, const void* k, int64_t k
                        const int32_t* cu_seqlens, const int32_t* seq_chunk0, int64_t total_chunks, int nseq,
                        int seq_len, int Hqk, int Hv, int D, int in_dtype, int use_qk_l2norm, void* workspace,
                        int64_t workspace_bytes, void* stream, const GateArgs& gate, int norm_mode,
-                       bool table_built = false, bool check_only = false) {
+                       bool table_built = false, bool check_only = false, const CaptureArgs& cap = CaptureArgs{}) {
   GDN_REQUIRE(state_rows ? n_rows >= 0 : n_rows == nseq,
               "gdn_chunk_prefill: without state_rows, n_rows must equal nseq");
   GDN_REQUIRE(q && k && v && g && beta && out, "gdn_chunk_prefill: null input/output pointer");
@@ -2136,15 +2153,15 @@ int chunk_prefill_impl(const void* q, int64_t q_stride, const void* k, int64_t k
                      (int)lay.L, walk};
   if (total_chunks > 0) {  // the intra-chunk inverses, one wave per (chunk, value head)
     const int64_t items = total_chunks * Hv;
-    const unsigned gi = (unsigned)((items + 3) / 4);
+    const unsigned gi = (unsigned)((items + 3) / 4 + cap.n);
     if (beta_dtype == GDN_BF16)
       inv_kernel<uint16_t><<<gi, pf::NT, 0, st>>>((const uint16_t*)k, k_stride, g,
                                                   (const uint16_t*)beta, cu_seqlens, seq_chunk0, nseq, seq_len, items,
-                                                  Hqk, Hv, use_qk_l2norm, tfrag, knorm, tab, warm);
+                                                  Hqk, Hv, use_qk_l2norm, tfrag, knorm, tab, warm, cap);
     else
       inv_kernel<float><<<gi, pf::NT, 0, st>>>((const uint16_t*)k, k_stride, g,
                                                (const float*)beta, cu_seqlens, seq_chunk0, nseq, seq_len, items, Hqk,
-                                               Hv, use_qk_l2norm, tfrag, knorm, tab, warm);
+                                               Hv, use_qk_l2norm, tfrag, knorm, tab, warm, cap);
     int rc = check_launch("gdn_chunk_prefill(inverse)");
     if (rc) return rc;
   }
@@ -2317,11 +2334,11 @@ extern "C" int gdn_chunk_prefill_inverse(const void* k, int64_t k_stride, const 
   if (beta_dtype == GDN_BF16)
     inv_kernel<uint16_t><<<gi, pf::NT, 0, st>>>((const uint16_t*)k, k_stride, g, (const uint16_t*)beta, cu_seqlens,
                                                 seq_chunk0, nseq, seq_len, items, Hqk, Hv, use_qk_l2norm, tfrag,
-                                                knorm, tab, warm);
+                                                knorm, tab, warm, CaptureArgs{});
   else
     inv_kernel<float><<<gi, pf::NT, 0, st>>>((const uint16_t*)k, k_stride, g, (const float*)beta, cu_seqlens,
                                              seq_chunk0, nseq, seq_len, items, Hqk, Hv, use_qk_l2norm, tfrag, knorm,
-                                             tab, warm);
+                                             tab, warm, CaptureArgs{});
   int rc = check_launch("gdn_chunk_prefill_inverse(inverse)");
   if (rc) return rc;
   inv_records_expand_kernel<<<gi, 256, 0, st>>>(tfrag, knorm, items, t_out, use_qk_l2norm ? factor_out : nullptr);
@@ -2458,12 +2475,13 @@ extern "C" int gdn_prefill_layer_rows(const void* mixed, int64_t mixed_stride, c
   uint16_t* conv_out = (uint16_t*)work;
   const GateArgs gate{(const uint16_t*)z, z_stride, norm_w, eps};
   const int64_t kd = (int64_t)Hk * D;
+  CaptureArgs cap{};
   auto rule = [&](bool check_only) {  // the chunked rule on the prologue's outputs
     return chunk_prefill_impl(conv_out, C, conv_out + kd, C, conv_out + 2 * kd, C, (float*)(work + lay.off_g),
                               work + lay.off_beta, GDN_BF16, initial_state, final_state, state_rows, n_rows, out,
                               total_tokens, cu_seqlens, seq_chunk0, total_chunks, nseq, seq_len, Hk, Hv, D, GDN_BF16,
                               1, work + lay.off_chunk, workspace_bytes - lay.off_chunk, stream, gate,
-                              norm_w_dtype == GDN_BF16 ? 1 : 2, cu_seqlens != nullptr, check_only);
+                              norm_w_dtype == GDN_BF16 ? 1 : 2, cu_seqlens != nullptr, check_only, cap);
   };
   // every check of the chunked rule runs before the first launch: a refusal leaves the conv state
   // and the slot rows untouched
@@ -2534,12 +2552,18 @@ extern "C" int gdn_prefill_layer_rows(const void* mixed, int64_t mixed_stride, c
     if (rc) return rc;
   }
   if (!cap_fused) {  // the history rows are the state rows: the capture reads them after the conv has
-    const int64_t n = (int64_t)nseq * C;
-    conv_state_capture_kernel<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(
-        (const uint16_t*)mixed, mixed_stride, (const uint16_t*)conv_history, state_rows, (uint16_t*)conv_state,
-        state_rows, n_rows, cu_seqlens, nseq, seq_len, C, K);
-    int rc = check_launch("gdn_prefill_layer(state)");
-    if (rc) return rc;
+    const int64_t n = ((int64_t)nseq * C + 255) / 256;
+    if (total_chunks > 0 && n < (1 << 20)) {
+      cap = CaptureArgs{(int)((n + 7) / 8 * 8), (const uint16_t*)mixed, mixed_stride, (uint16_t*)conv_state, state_rows,
+                        n_rows, C, K};
+    } else {
+      conv_state_capture_kernel<<<(unsigned)n, 256, 0, st>>>((const uint16_t*)mixed, mixed_stride,
+                                                             (const uint16_t*)conv_history, state_rows,
+                                                             (uint16_t*)conv_state, state_rows, n_rows, cu_seqlens,
+                                                             nseq, seq_len, C, K);
+      const int rc = check_launch("gdn_prefill_layer(state)");
+      if (rc) return rc;
+    }
   }
   return rule(false);
 }
