@@ -101,9 +101,14 @@ def exported_symbols():
     return [n for n in _SIGNATURES if getattr(h, n, None) is not None]
 
 
+_entries = {}  # name -> bound entry point of the loaded library
+
+
 def call(name, *args):
     """Call a C-ABI entry point; raise GDNError with the library's message on failure."""
-    fn = getattr(lib(), name)
+    fn = _entries.get(name)
+    if fn is None:
+        fn = _entries[name] = getattr(lib(), name)
     rc = fn(*args)
     if rc != 0:
         msg = lib().gdn_last_error().decode(errors="replace")
@@ -113,31 +118,34 @@ def call(name, *args):
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
+# Pointers and streams go to the entry points as plain ints (None: null), which a c_void_p argument takes
+# directly: a c_void_p object per argument costs a small call about a microsecond of host time in all.
 def stream_of(t):
     """Raw hipStream_t of torch's current stream on t's device (torch's raw-handle query when it has
     one: no Stream object per call)."""
     if _raw_stream is not None:
-        return ctypes.c_void_p(_raw_stream(t.get_device()))
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+        return _raw_stream(t.get_device())
+    return torch.cuda.current_stream(t.device).cuda_stream
 
 
 def ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
-
-
-def ptr_int(t):
-    """Device address as a plain int (None for None): what a c_void_p argument takes directly."""
+    """Device address of a tensor (None for None)."""
     return None if t is None else t.data_ptr()
 
 
+_CODES = {torch.float32: F32, torch.bfloat16: BF16, torch.float16: F16}
+
+
 def dtype_code(t):
-    if t.dtype == torch.float32:
-        return F32
-    if t.dtype == torch.bfloat16:
-        return BF16
-    if t.dtype == torch.float16:
-        return F16
-    raise TypeError(f"unsupported dtype {t.dtype} (float32, bfloat16 or float16)")
+    code = _CODES.get(t.dtype)
+    if code is None:
+        raise TypeError(f"unsupported dtype {t.dtype} (float32, bfloat16 or float16)")
+    return code
+
+
+def f32_dense(t):
+    """t as a contiguous fp32 tensor (itself when it is one)."""
+    return t if t.dtype == torch.float32 and t.is_contiguous() else t.to(torch.float32).contiguous()
 
 
 def dense_rows(t):

@@ -35,7 +35,7 @@ def elem_conv_update(x, state, weight, bias):
     if T != 1:
         raise ValueError("elem_conv_update: one token per call (x [n,C,1])")
     K = weight.shape[-1]
-    if tuple(state.shape) != (n, C, K) or tuple(weight.shape) != (C, K):
+    if state.shape != (n, C, K) or weight.shape != (C, K):
         raise ValueError(f"elem_conv_update: state {tuple(state.shape)} / weight {tuple(weight.shape)} "
                          f"do not match x {tuple(x.shape)}")
     if not (x.dtype == state.dtype == weight.dtype == torch.bfloat16):
@@ -44,11 +44,13 @@ def elem_conv_update(x, state, weight, bias):
         raise ValueError("elem_conv_update: state must be contiguous (it is updated in place)")
     if bias is not None:
         bias = bias.to(torch.bfloat16).contiguous()
-    weight = weight.contiguous()
-    xr, xs = _row_view(x[:, :, 0])
-    out = torch.empty(n, C, 1, dtype=x.dtype, device=x.device)
-    _lib.call("gdn_conv_update", _lib.ptr(xr), xs, _lib.ptr(state), _lib.ptr(weight), _lib.ptr(bias),
-              _lib.ptr(out), C, n, C, K, _lib.stream_of(x))
+    if not weight.is_contiguous():
+        weight = weight.contiguous()
+    if x.stride(1) != 1:                     # rows of C values; the token dimension's stride is never used
+        x = x[:, :, 0].contiguous().unsqueeze(-1)
+    out = torch.empty((n, C, 1), dtype=x.dtype, device=x.device)
+    _lib.call("gdn_conv_update", x.data_ptr(), x.stride(0), state.data_ptr(), weight.data_ptr(), _lib.ptr(bias),
+              out.data_ptr(), C, n, C, K, _lib.stream_of(x))
     return out
 
 
@@ -73,12 +75,12 @@ def gated_rmsnorm(hidden_states, gate, weight, eps=1e-6):
     D = hidden_states.shape[-1]
     if gate.shape != hidden_states.shape or weight.shape != (D,):
         raise ValueError("gated_rmsnorm: gate must match hidden_states and weight must be [D]")
-    x, xs = _row_view(hidden_states.reshape(-1, D))
-    z, zs = _row_view(gate.reshape(-1, D))
-    w = weight.contiguous()
-    out = torch.empty(hidden_states.shape, dtype=hidden_states.dtype, device=hidden_states.device)
-    _lib.call("gdn_gated_rmsnorm", _lib.ptr(x), xs, _lib.ptr(z), zs, _lib.ptr(w), _lib.dtype_code(w),
-              _lib.ptr(out), x.shape[0], D, float(eps), _lib.stream_of(x))
+    x, xs = _row_view(hidden_states if hidden_states.dim() == 2 else hidden_states.reshape(-1, D))
+    z, zs = _row_view(gate if gate.dim() == 2 else gate.reshape(-1, D))
+    w = weight if weight.is_contiguous() else weight.contiguous()
+    out = torch.empty(hidden_states.shape, dtype=torch.bfloat16, device=x.device)
+    _lib.call("gdn_gated_rmsnorm", x.data_ptr(), xs, z.data_ptr(), zs, w.data_ptr(), _lib.dtype_code(w),
+              out.data_ptr(), x.shape[0], D, float(eps), _lib.stream_of(x))
     return out
 
 

@@ -23,16 +23,15 @@ from . import _lib
 CHUNK = 64
 
 
-def _tokens_view(x, name):
-    """[B, T, H, d] -> ([B*T, H, d] tensor with dense (H, d), token stride).  torch gives a size-1
-    dimension an arbitrary stride: a single token's stride is never used, a single head's is d."""
+def _token_rows(x):
+    """[B, T, H, d] as B T rows of dense (H, d): (x itself or a dense copy, token stride).  torch gives a
+    size-1 dimension an arbitrary stride: a single token's stride is never used, a single head's is d."""
     B, T, H, D = x.shape
-    ts = x.stride(1) if T > 1 else (x.stride(0) if B > 1 else H * D)
-    hs = x.stride(2) if H > 1 else D
-    if x.stride(3) != 1 or hs != D or (B > 1 and T > 1 and x.stride(0) != T * ts):
-        x, ts = x.clone(memory_format=torch.contiguous_format), H * D
-    flat = x.as_strided((B * T, H, D), (ts, D, 1))
-    return flat, ts
+    sb, st, sh, sd = x.stride()
+    ts = st if T > 1 else (sb if B > 1 else H * D)
+    if sd != 1 or (H > 1 and sh != D) or (B > 1 and T > 1 and sb != T * ts):
+        return x.clone(memory_format=torch.contiguous_format), H * D
+    return x, ts
 
 
 def _to_device_int32(host, device):
@@ -183,10 +182,10 @@ def chunk_gated_delta_rule(query, key, value, g, beta, chunk_size=64, initial_st
         cu, seq_chunk0, nseq, seq_len, total_chunks = _chunk_table(B, T, cu_seqlens, dev)
     else:  # the generic kernels number chunks by sequence: no chunk table, but the lengths' bound
         cu, _, nseq, seq_len, _ = _chunk_table(B, T, cu_seqlens, dev)
-    q, qs = _tokens_view(query, "query")
-    k, ks = _tokens_view(key, "key")
-    v, vs = _tokens_view(value, "value")
-    g32 = g.to(torch.float32).contiguous()
+    q, qs = _token_rows(query)
+    k, ks = _token_rows(key)
+    v, vs = _token_rows(value)
+    g32 = _lib.f32_dense(g)
     if beta.dtype not in ((torch.float32, torch.bfloat16) if fast else FLOATS):
         beta = beta.to(torch.float32)
     beta = beta.contiguous()
@@ -207,7 +206,7 @@ def chunk_gated_delta_rule(query, key, value, g, beta, chunk_size=64, initial_st
         if initial_state is not None:
             if tuple(initial_state.shape) != (nseq, Hv, D, Dv):
                 raise ValueError(f"chunk_gated_delta_rule: initial_state must be [{nseq},{Hv},{D},{Dv}]")
-            init = initial_state.to(torch.float32).contiguous()
+            init = _lib.f32_dense(initial_state)
         final = torch.empty(nseq, Hv, D, Dv, dtype=torch.float32, device=dev) if output_final_state else None
     out = torch.empty(B, T, Hv, Dv, dtype=query.dtype, device=dev)
     if not fast:
@@ -278,7 +277,7 @@ def chunk_inverse_records(key, g, beta, use_qk_l2norm_in_kernel=True, cu_seqlens
         raise ValueError("chunk_inverse_records: g, beta must be [B, T, Hv] with Hv a multiple of Hk")
     dev = key.device
     cu, seq_chunk0, nseq, seq_len, total_chunks = _chunk_table(B, T, cu_seqlens, dev)
-    k, ks = _tokens_view(key, "key")
+    k, ks = _token_rows(key)
     g32 = g.to(torch.float32).contiguous()
     if beta.dtype not in (torch.float32, torch.bfloat16):
         beta = beta.to(torch.float32)
@@ -348,16 +347,18 @@ def gdn_gating(a, b, A_log, dt_bias):
     (src/cb_engine.py:337-338).  a, b [..., Hv] bf16."""
     _lib.require_cuda(a, b)
     Hv = a.shape[-1]
-    a2 = a.reshape(-1, Hv)
-    b2 = b.reshape(-1, Hv)
+    a2 = a if a.dim() == 2 else a.reshape(-1, Hv)
+    b2 = b if b.dim() == 2 and b.shape[1] == Hv else b.reshape(-1, Hv)
+    if a.numel() != b.numel():
+        raise ValueError(f"gdn_gating: a {tuple(a.shape)} and b {tuple(b.shape)} hold different numbers of values")
     if a2.stride() != b2.stride() or a2.stride(-1) != 1:
         a2, b2 = a2.contiguous(), b2.contiguous()
-    beta = torch.empty(a2.shape, dtype=torch.bfloat16, device=a.device)
-    g = torch.empty(a2.shape, dtype=torch.float32, device=a.device)
-    _lib.call("gdn_gating", _lib.ptr(a2), _lib.ptr(b2), a2.stride(0),
-              _lib.ptr(A_log.to(torch.float32).contiguous()), _lib.ptr(dt_bias.to(torch.float32).contiguous()),
-              _lib.ptr(beta), _lib.ptr(g), a2.shape[0], Hv, _lib.stream_of(a))
-    return beta.reshape(b.shape), g.reshape(a.shape)
+    A32, dt32 = _lib.f32_dense(A_log), _lib.f32_dense(dt_bias)
+    beta = torch.empty(b.shape, dtype=torch.bfloat16, device=a.device)
+    g = torch.empty(a.shape, dtype=torch.float32, device=a.device)
+    _lib.call("gdn_gating", a2.data_ptr(), b2.data_ptr(), a2.stride(0), A32.data_ptr(), dt32.data_ptr(),
+              beta.data_ptr(), g.data_ptr(), a2.shape[0], Hv, _lib.stream_of(a))
+    return beta, g
 
 
 def gdn_prefill_core(mixed_qkv, z, a, b, conv_weight, A_log, dt_bias, norm_weight, num_k_heads,
@@ -460,7 +461,7 @@ def gdn_prefill_core(mixed_qkv, z, a, b, conv_weight, A_log, dt_bias, norm_weigh
     core = torch.empty(T, Hv * D, dtype=torch.bfloat16, device=dev)
     wbytes = int(_lib.lib().gdn_prefill_layer_workspace_bytes(T, total_chunks, nseq, Hk, Hv, D))
     work = torch.empty(max(wbytes, 1), dtype=torch.uint8, device=dev)
-    p = _lib.ptr_int
+    p = _lib.ptr
     _lib.call("gdn_prefill_layer_rows", x.data_ptr(), xs, z2.data_ptr(), zs, a2.data_ptr(),
               b2.data_ptr(), ab_rs, w.data_ptr(), p(bias), A32.data_ptr(), dt32.data_ptr(), nw.data_ptr(),
               _lib.dtype_code(nw), float(eps), p(hist), conv_state.data_ptr(), p(init), rec.data_ptr(),

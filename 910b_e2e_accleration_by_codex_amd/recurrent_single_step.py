@@ -13,23 +13,11 @@ import torch
 from . import _lib
 
 
-def _rows(x):
-    """[N, H, D] view whose H and D are dense; returns (tensor, row stride)."""
-    if x.stride(-1) != 1 or x.stride(-2) != x.shape[-1]:
+def _head_rows(x):
+    """[N, T, H, D] as rows of H D values: (tensor whose H and D are dense, slot stride, token stride)."""
+    if x.stride(3) != 1 or x.stride(2) != x.shape[3]:
         x = x.contiguous()
-    return x, x.stride(0)
-
-
-def _step(q, k, v, g, beta, state_in, state_out, out, use_l2):
-    """q,k [N,Hqk,D], v [N,Hv,D], g [N,Hv] fp32, beta [N,Hv], out [N,Hv,D] (dense)."""
-    N, Hqk, D = q.shape
-    Hv = v.shape[1]
-    q, qs = _rows(q)
-    k, ks = _rows(k)
-    v, vs = _rows(v)
-    _lib.call("gdn_recurrent_step", _lib.ptr(q), qs, _lib.ptr(k), ks, _lib.ptr(v), vs, _lib.ptr(g),
-              _lib.ptr(beta), _lib.dtype_code(beta), _lib.ptr(state_in), _lib.ptr(state_out),
-              _lib.ptr(out), N, Hqk, Hv, D, _lib.dtype_code(q), int(bool(use_l2)), _lib.stream_of(q))
+    return x, x.stride(0), x.stride(1)
 
 
 def recurrent_single_step(query, key, value, g, beta, initial_state, output_final_state,
@@ -47,34 +35,43 @@ def recurrent_single_step(query, key, value, g, beta, initial_state, output_fina
     if key.shape != query.shape or value.shape[:2] != (N, T) or value.shape[3] != D:
         raise ValueError(f"recurrent_single_step: shape mismatch q{tuple(query.shape)} "
                          f"k{tuple(key.shape)} v{tuple(value.shape)}")
-    if tuple(g.shape) != (N, T, Hv) or tuple(beta.shape) != (N, T, Hv):
+    if g.shape != (N, T, Hv) or beta.shape != (N, T, Hv):
         raise ValueError("recurrent_single_step: g and beta must be [N, T, Hv]")
-    g = g.to(torch.float32)
+    if g.dtype != torch.float32:
+        g = g.to(torch.float32)
     if beta.dtype not in (torch.float32, torch.bfloat16):
         beta = beta.to(torch.float32)
     state_in = None
     if initial_state is not None:
-        if tuple(initial_state.shape) != (N, Hv, D, D):
+        if initial_state.shape != (N, Hv, D, D):
             raise ValueError(f"recurrent_single_step: state must be [{N},{Hv},{D},{D}]")
         if inplace and (initial_state.dtype != torch.float32 or not initial_state.is_contiguous()):
             raise ValueError("recurrent_single_step: inplace needs a contiguous fp32 state")
-        state_in = initial_state if (initial_state.dtype == torch.float32
-                                     and initial_state.is_contiguous()) else \
-            initial_state.to(torch.float32).contiguous()
+        state_in = _lib.f32_dense(initial_state)
+    dev = query.device
     if inplace and initial_state is not None:
         state_out = state_in
     else:
-        state_out = torch.empty(N, Hv, D, D, dtype=torch.float32, device=query.device)
-    out = torch.empty(N, T, Hv, D, dtype=query.dtype, device=query.device)
+        state_out = torch.empty((N, Hv, D, D), dtype=torch.float32, device=dev)
+    out = torch.empty((N, T, Hv, D), dtype=query.dtype, device=dev)
+    q, qn, qt = _head_rows(query)
+    k, kn, kt = _head_rows(key)
+    v, vn, vt = _head_rows(value)
+    flags = (Hqk, Hv, D, _lib.dtype_code(query), int(bool(use_qk_l2norm_in_kernel)), _lib.stream_of(query))
+    bcode = _lib.dtype_code(beta)
     if T == 1:
-        _step(query[:, 0], key[:, 0], value[:, 0], g[:, 0].contiguous(), beta[:, 0].contiguous(),
-              state_in, state_out, out[:, 0], use_qk_l2norm_in_kernel)
+        g, beta = g.contiguous(), beta.contiguous()
+        _lib.call("gdn_recurrent_step", q.data_ptr(), qn, k.data_ptr(), kn, v.data_ptr(), vn, g.data_ptr(),
+                  beta.data_ptr(), bcode, _lib.ptr(state_in), state_out.data_ptr(), out.data_ptr(), N, *flags)
     else:
+        es = q.element_size()
         cur = state_in
-        step_out = torch.empty(N, Hv, D, dtype=query.dtype, device=query.device)
+        step_out = torch.empty((N, Hv, D), dtype=query.dtype, device=dev)
         for t in range(T):
-            _step(query[:, t], key[:, t], value[:, t], g[:, t].contiguous(), beta[:, t].contiguous(),
-                  cur, state_out, step_out, use_qk_l2norm_in_kernel)
+            gt, bt = g[:, t].contiguous(), beta[:, t].contiguous()
+            _lib.call("gdn_recurrent_step", q.data_ptr() + t * qt * es, qn, k.data_ptr() + t * kt * es, kn,
+                      v.data_ptr() + t * vt * es, vn, gt.data_ptr(), bt.data_ptr(), bcode, _lib.ptr(cur),
+                      state_out.data_ptr(), step_out.data_ptr(), N, *flags)
             out[:, t].copy_(step_out)
             cur = state_out
     return out, (state_out if output_final_state else None)
