@@ -286,6 +286,7 @@ struct SegTable {
   const int32_t* seg0;
   const int32_t* order;  // output pass: segments longest first (nullptr: in index order)
   int nseq, seq_len, L;
+  int balance;  // the output pass evens its segments out over the heads' warm-ups (plan_segments)
   int walk;  // pairs without warm-ups walk their whole sequence in one workgroup (no summary pass): walk_pays()
   __device__ __forceinline__ int nch(int s) const {
     return cu ? chunk0[s + 1] - chunk0[s] : (seq_len + pf::CH - 1) / pf::CH;
@@ -404,9 +405,11 @@ __global__ __launch_bounds__(256) void seg_table_kernel(const int32_t* __restric
 // keeps everything in registers: no LDS round trips of intermediate products and no barriers.
 typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
 // The inverse kernel's second record per (chunk, value head): the K rows' l2norm factors, the chunk's
-// g values (both fp32, by token) and a flag word (nonzero: the T record's lo part was written).
+// g values (both fp32, by token), a flag word (nonzero: the T record's lo part was written) and the
+// chunk's summed g.
 namespace kr {
 constexpr int FLAG = 2 * pf::CH;      // float index of the flag word
+constexpr int SUM = FLAG + 1;         // the chunk's summed g, NaN where the warm-up bound does not hold in it
 constexpr int FLOATS = 2 * pf::CH + 4;  // 528 bytes: 16-byte aligned records
 }  // namespace kr
 namespace tf {
@@ -652,8 +655,15 @@ __global__ __launch_bounds__(pf::NT, 2) void inv_kernel(const uint16_t* __restri
   bool lo_rec = __expf(Gl) > sg::kPreciseGl || Gl > sg::kLoRecordLog;
   if (!lo_rec)
     lo_rec = tail_decay_above(g, Hv, h, t_tail, t_end, sg::kLoRecordLog, gtail);
-  if (lane == 0)
-    reinterpret_cast<int*>(knorm)[((int64_t)slot * Hv + h) * kr::FLOATS + kr::FLAG] = lo_rec ? 1 : 0;
+  {  // (a NaN in g makes the sum one)
+    const float b = sdec[w][1][lane];
+    const bool ok = use_l2 && __builtin_amdgcn_ballot_w64(!(b >= 0.f && b <= 1.f)) == 0;
+    if (lane == 0) {
+      float* rec = knorm + ((int64_t)slot * Hv + h) * kr::FLOATS;
+      reinterpret_cast<int*>(rec)[kr::FLAG] = lo_rec ? 1 : 0;
+      rec[kr::SUM] = ok ? Gl : __builtin_nanf("");
+    }
+  }
   // fragments (w', s), s <= w' / 2: element e of lane (i, g) = T[16 w' + i][j] beta_j with
   // j = 32 s + kpos(8 g + e), kpos(8 g + e) = 16 (e >> 2) + 4 g + (e & 3): blocks 2s (e < 4) and 2s + 1
   uint8_t* dst = tfrag + ((int64_t)slot * Hv + h) * tf::BYTES;
@@ -726,6 +736,128 @@ __device__ bool seq_warm_ok(const SegTable& tab, const int* __restrict__ warm, i
     if (__builtin_amdgcn_ballot_w64(wv == 0) != 0) return false;
   }
   return true;
+}
+
+// Balanced segments.  With L chunks a segment, a head whose warm-ups take w chunks runs L + w steps a segment,
+// and the slowest head sets the output pass's time (T = 32768 with heads of every memory length: 64 + 28
+// steps where the mean is 70).  The output pass therefore takes the least number of steps T such that segments
+// of T chunks (a sequence's first) and T - w (the others) need at most kTargetItems workgroups over all
+// (sequence, key head) groups, w = the largest of the group's warm-ups at the fixed segments' ends; groups
+// with a head on the exact path keep their fixed segments.  (Per group, not per value head: the value
+// heads of a key head then still run the same chunks side by side and share its q and K in L2.)  Every
+// workgroup works it out from the warm-up lengths by itself (about 1 us).
+constexpr int kMaxGroups = sg::kTargetItems;  // nseq Hqk <= nseq Hv <= kTargetItems
+constexpr int kBalanceMin = 24;
+struct PlanSmem {
+  int w[kMaxGroups], n[kMaxGroups];  // the group's warm-up (kExactGroup: fixed segments) and its chunks
+  int best, s, hk, local, cnt;       // the step count found; this workgroup's group and place in it
+};
+constexpr int kExactGroup = 1 << 30;
+struct PlanItem {
+  bool on;        // false: the fixed segments stand
+  bool idle;      // on, and no item is left for this workgroup
+  int s, h;
+  int begin, end;  // chunks; end < 0: fixed segment number `begin` of a group on the exact path
+};
+// A group with warm-ups of 3 or more chunks forgets less than e^-4 a chunk: its steps take W S in hi + lo and
+// cost 4/3 of the others (T = 8192: 5.2 against 4.0 us), so it runs 3/4 as many.
+__device__ __forceinline__ int plan_steps(int w, int steps) { return w >= 3 ? 3 * steps / 4 : steps; }
+// Segments of a group of n chunks at `steps` steps, or a number past every target.
+__device__ __forceinline__ int plan_count(int n, int w, int steps, int L) {
+  if (w == kExactGroup) return n <= L ? 1 : (n + L - 1) / L;
+  steps = plan_steps(w, steps);
+  if (n <= steps) return 1;
+  const int d = steps - w;
+  return d < 1 ? sg::kTargetItems + 1 : 1 + (n - steps + d - 1) / d;
+}
+__device__ PlanItem plan_segments(PlanSmem& P, const SegTable& tab, const int* __restrict__ warm, int Hqk, int Hv, int b) {
+  const int t = threadIdx.x, r = Hv / Hqk, groups = tab.nseq * Hqk, entries = tab.first_slot(tab.nseq) * Hv;
+  if (t < groups) {
+    const int n = tab.nch(t / Hqk);
+    P.n[t] = n;
+    P.w[t] = n <= tab.L ? kExactGroup : 0;  // (nothing known of its warm-ups: one fixed segment)
+  }
+  if (t == 0) P.best = kExactGroup, P.cnt = 0;
+  __syncthreads();
+  for (int e = t; e < entries; e += sg::NT) {
+    const int wv = warm[e];
+    atomicMax(&P.w[tab.seq_of_slot(e / Hv) * Hqk + (e % Hv) / r], wv == 0 ? kExactGroup : wv);
+  }
+  __syncthreads();
+  // candidates: from an even share up to what the fixed segments take
+  int64_t chunks = 0;
+  int wmax = 0, fixed = 0;
+  for (int i = 0; i < groups; ++i) {
+    const int n = P.n[i], w = P.w[i];
+    chunks += n;
+    if (w != kExactGroup) wmax = w > wmax ? w : wmax;
+    else fixed = n >= tab.L ? tab.L : n > fixed ? n : fixed;
+  }
+  int lo = (int)((chunks * r + sg::kTargetItems - 1) / sg::kTargetItems);
+  lo = lo > fixed ? lo : fixed;
+  // warm-ups of a sixteenth of a segment: nothing to even out
+  const int hi = 16 * wmax <= tab.L ? 0 : (tab.L + wmax) * 4 / 3;
+  if (__builtin_amdgcn_readfirstlane(hi) == 0) {
+    __syncthreads();
+    return PlanItem{false, false, 0, 0, 0, 0};
+  }
+  const int by = (hi - lo + sg::NT - 1) / sg::NT;
+  const int steps = lo + t * (by < 1 ? 1 : by);
+  if (steps > 0 && steps < hi) {
+    int sum = 0;
+    for (int i = 0; i < groups && sum <= sg::kTargetItems; ++i) sum += r * plan_count(P.n[i], P.w[i], steps, tab.L);
+    if (sum <= sg::kTargetItems) atomicMin(&P.best, steps);
+  }
+  __syncthreads();
+  PlanItem it{false, false, 0, 0, 0, 0};
+  const int T = __builtin_amdgcn_readfirstlane(P.best);
+  if (T != kExactGroup) {
+    it.on = true;
+    if (t < groups) {
+      int base = 0;
+      for (int i = 0; i < t; ++i) base += r * plan_count(P.n[i], P.w[i], T, tab.L);
+      const int c = r * plan_count(P.n[t], P.w[t], T, tab.L);
+      if (b >= base && b < base + c) {
+        P.s = t / Hqk;
+        P.hk = t % Hqk;
+        P.local = b - base;
+        P.cnt = c;
+      }
+    }
+    __syncthreads();
+    it.idle = __builtin_amdgcn_readfirstlane(P.cnt) == 0;
+    if (!it.idle) {  // (wave-uniform values: scalar addresses and branches in the chunk loop)
+      it.s = __builtin_amdgcn_readfirstlane(P.s);
+      const int hk = __builtin_amdgcn_readfirstlane(P.hk), local = __builtin_amdgcn_readfirstlane(P.local);
+      const int n = __builtin_amdgcn_readfirstlane(P.n[it.s * Hqk + hk]), w = __builtin_amdgcn_readfirstlane(P.w[it.s * Hqk + hk]);
+      const int i = local / r;
+      it.h = hk * r + local % r;
+      const int Tg = plan_steps(w, T);
+      it.begin = i == 0 ? 0 : Tg + (i - 1) * (Tg - w);
+      it.end = i == 0 ? Tg : it.begin + Tg - w;
+      if (it.end > n) it.end = n;
+      if (w == kExactGroup) it.begin = i, it.end = -1;
+    }
+  }
+  __syncthreads();  // the caller's chunk buffers take this memory
+  return it;
+}
+// The least number of chunks before chunk c of sequence s (head h) whose summed log decay is below
+// kWarmLog, or c when there is none before the sequence's start (one wave; sums from the inverse
+// kernel's records, 64 chunks at a time).
+__device__ int warm_before(const SegTable& tab, const float* __restrict__ knorm, int Hv, int h, int s, int c) {
+  const int lane = threadIdx.x & 63;
+  const int64_t first = tab.first_chunk(s);
+  float acc = 0.f;
+  for (int c0 = 0; c0 < c; c0 += 64) {
+    const int back = c0 + lane;  // chunk c - 1 - back
+    const float x = back < c ? knorm[((first + c - 1 - back) * Hv + h) * kr::FLOATS + kr::SUM] : 0.f;
+    const float sum = acc + wave_incl_scan(x);
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(back < c && sum < sg::kWarmLog);
+    if (hit) return c0 + __builtin_ctzll(hit) + 1;
+    acc = __shfl(sum, 63, kWave);
+  }
+  return c;
 }
 
 // Work item of workgroup b of n: workgroups are dealt to the 8 XCDs round-robin (b % 8), so items
@@ -1343,17 +1475,28 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
     const int* __restrict__ warm, GateArgs gate) {
   using namespace pf;
   __shared__ SegSmem sm;
+  static_assert(sizeof(SegSmem) >= sizeof(PlanSmem), "the plan sits in the chunk buffers");
   static_assert(sizeof(SegSmem) >= (size_t)D * kALd * 4 && sizeof(SegSmem) >= 2 * 64 * ws::FRAG,
                 "the chunk buffers hold A_j's row-major copy and two slots' A fragments");
   const int t = threadIdx.x, w = t >> 6, lane = t & 63, c16 = lane & 15, g4 = lane >> 4;
   int mode, h, s, idx, slot = -1;
+  PlanItem plan{false, false, 0, 0, 0, 0};
   if (kPass == 0) {
-    const int item = xcd_item(blockIdx.x, gridDim.x), jo = item / Hv;
-    h = item % Hv;
-    if (jo >= tab.first_seg(tab.nseq)) return;
-    const int j = tab.order ? tab.order[jo] : jo;
-    s = tab.seq_of_seg(j);
-    idx = j - tab.first_seg(s);
+    const int item = xcd_item(blockIdx.x, gridDim.x);
+    if (tab.balance) plan = plan_segments(reinterpret_cast<PlanSmem&>(sm), tab, warm, Hqk, Hv, item);
+    if (plan.on) {
+      if (plan.idle) return;
+      s = plan.s;
+      h = plan.h;
+      idx = plan.end < 0 ? plan.begin : 0;
+    } else {
+      const int jo = item / Hv;
+      h = item % Hv;
+      if (jo >= tab.first_seg(tab.nseq)) return;
+      const int j = tab.order ? tab.order[jo] : jo;
+      s = tab.seq_of_seg(j);
+      idx = j - tab.first_seg(s);
+    }
     if (idx > 0) slot = tab.first_slot(s) + idx - 1;  // the previous segment's slot holds this one's state
     mode = kSegOut;
   } else {
@@ -1378,8 +1521,9 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
   const int combine_steps = (kPass == 0 && slot >= 0 && !warm_path) ? idx : 0;
   const int ts_first = tab.first_slot(s);
   const int kh = h / (Hv / Hqk);
-  const int c_begin = idx * tab.L;
-  const int n = walk || nch_s - c_begin < tab.L ? nch_s - c_begin : tab.L;
+  const bool even = plan.on && plan.end >= 0;  // a balanced segment: its own chunk range, warm-up or initial state
+  const int c_begin = even ? plan.begin : idx * tab.L;
+  const int n = even ? plan.end - plan.begin : walk || nch_s - c_begin < tab.L ? nch_s - c_begin : tab.L;
   const int64_t t_seq = tab.start(s);
   const int Ls = tab.len(s);
   float* tslot = slot >= 0 ? trans + ((int64_t)slot * Hv + h) * sg::kTrans : nullptr;
@@ -1409,7 +1553,8 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
   }
   constexpr bool need_q = kPass == 0;
   // pass 0 after a warm-up: the chain starts from zero w0 chunks before the segment, without outputs
-  const int w0 = (kPass == 0 && warm_path) ? warm[(int64_t)slot * Hv + h] : 0;
+  const int w0 = even ? (c_begin > 0 ? warm_before(tab, knorm, Hv, h, s, c_begin) : 0)
+                      : (kPass == 0 && warm_path) ? warm[(int64_t)slot * Hv + h] : 0;
   const int cb0 = c_begin - w0, ntot = n + w0;
   const int chunk_slot0 = tab.first_chunk(s) + cb0;
   auto tfr = [&](int c) { return tfrag + ((int64_t)(chunk_slot0 + c) * Hv + h) * tf::BYTES; };
@@ -1567,7 +1712,7 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
     ChainRegs R;
     {  // initial state: the sequence's (then, on the exact path, the combination below), or zero
       const float* src = nullptr;
-      if (mode == kSegOut && (slot < 0 || !warm_path) && init) {
+      if (mode == kSegOut && (even ? cb0 == 0 : slot < 0 || !warm_path) && init) {
         const int r0 = state_row(rows, n_rows, s);
         if (r0 >= 0) src = init + ((int64_t)r0 * Hv + h) * D * D;
       }
@@ -1674,7 +1819,7 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
     }
     // the state after the segment
     if (mode == kSegOut) {
-      if (final_state && (walk || idx == nseg_s - 1)) {
+      if (final_state && (even ? c_begin + n == nch_s : walk || idx == nseg_s - 1)) {
         const int r0 = state_row(rows, n_rows, s);
         if (r0 >= 0) {
           float* dst = final_state + ((int64_t)r0 * Hv + h) * D * D;
@@ -2149,8 +2294,11 @@ int chunk_prefill_impl(const void* q, int64_t q_stride, const void* k, int64_t k
   // packed sequences an upper bound of the longest one (0: unknown)
   const int64_t max_seq_chunks = seq_len > 0 ? ((int64_t)seq_len + pf::CH - 1) / pf::CH : total_chunks;
   const int walk = walk_pays(max_seq_chunks, lay, Hv, norm_mode != 0) ? 1 : 0;
+  // segments evened out over the heads' warm-ups: where one round of workgroups holds them all and a segment is
+  // long enough for the heads to differ by more than the planning costs
+  const int balance = !walk && max_seq_chunks > lay.L && lay.L >= kBalanceMin && (int64_t)nseq * Hv <= sg::kTargetItems;
   const SegTable tab{cu_seqlens, seq_chunk0, cu_seqlens ? seg0 : nullptr, cu_seqlens ? order : nullptr, nseq, seq_len,
-                     (int)lay.L, walk};
+                     (int)lay.L, balance, walk};
   if (total_chunks > 0) {  // the intra-chunk inverses, one wave per (chunk, value head)
     const int64_t items = total_chunks * Hv;
     const unsigned gi = (unsigned)((items + 3) / 4 + cap.n);
@@ -2183,7 +2331,7 @@ int chunk_prefill_impl(const void* q, int64_t q_stride, const void* k, int64_t k
     int rc = check_launch("gdn_chunk_prefill(summary)");
     if (rc) return rc;
   }
-  launch(0, nseg_max * Hv);
+  launch(0, balance && nseg_max * Hv < sg::kTargetItems ? sg::kTargetItems : nseg_max * Hv);
   return check_launch("gdn_chunk_prefill(output)");
 }
 }  // namespace
@@ -2325,7 +2473,7 @@ extern "C" int gdn_chunk_prefill_inverse(const void* k, int64_t k_stride, const 
     const int rc = check_launch("gdn_chunk_prefill_inverse(table)");
     if (rc) return rc;
   }
-  const SegTable tab{cu_seqlens, seq_chunk0, cu_seqlens ? seg0 : nullptr, nullptr, nseq, seq_len, (int)lay.L, 0};
+  const SegTable tab{cu_seqlens, seq_chunk0, cu_seqlens ? seg0 : nullptr, nullptr, nseq, seq_len, (int)lay.L, 0, 0};
   uint8_t* tfrag = work + lay.off_tfrag;
   float* knorm = (float*)(work + lay.off_knorm);
   int* warm = (int*)(work + lay.off_warm);

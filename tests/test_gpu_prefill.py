@@ -495,3 +495,34 @@ def test_chunk_prefill_short_sequences_walk(gdn, oracle, dev, lens, n_rows):
             assert rel_l2(sd[rows[i], h], s_ref[i, h]) <= STATE_TOL, (i, h)
     for spare in set(range(n_rows)) - set(rows):
         assert torch.equal(sd[spare].cpu(), slots[spare])
+
+
+@pytest.mark.parametrize("lens,Hk,Hv,exact", [([16447], 16, 32, False), ([20000, 9000, 0, 3000], 8, 16, True),
+                                              ([16384], 8, 16, True)])
+def test_chunk_prefill_balanced_segments(gdn, oracle, dev, lens, Hk, Hv, exact):
+    """Heads of very different memory lengths in segments long enough to be evened out over their warm-ups
+    (1 to about 20 chunks): some groups run more, shorter segments than others; with `exact`, one head has no
+    warm-up at all and another a beta above 1 (a segment near it starts from the sequence's start), beside heads of
+    the same key head that warm up.  Initial states; every (sequence, head) against the oracle."""
+    T = sum(lens)
+    q, k, v, g, beta, _ = _gdn_inputs(T, Hk, Hv, seed=T + Hv, state=False)
+    g *= torch.logspace(-1.3, 1, Hv)
+    if exact:
+        g[..., 3] *= 0.001
+        beta[0, 5000, Hv - 1] = 1.5
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    s0 = 0.02 * torch.randn(len(lens), Hv, 128, 128, generator=torch.Generator().manual_seed(6))
+    r = Hv // Hk
+    o_ref, s_ref = oracle.chunk_gated_delta_rule_varlen(_rep(q, r), _rep(k, r), v, g, beta, torch.tensor(cu), 64, s0,
+                                                        True, True)
+    o, s = gdn.chunk_gated_delta_rule(q.to(dev), k.to(dev), v.to(dev), g.to(dev), beta.to(dev), initial_state=s0.to(dev),
+                                      output_final_state=True, cu_seqlens=cu, use_qk_l2norm_in_kernel=True)
+    o, s = o.cpu(), s.cpu()
+    for i in range(len(lens)):
+        for h in range(Hv):
+            if lens[i]:
+                sl = slice(cu[i], cu[i + 1])
+                assert rel_l2(o[:, sl, h], o_ref[:, sl, h]) <= OUT_TOL, (i, h)
+            assert rel_l2(s[i, h], s_ref[i, h]) <= STATE_TOL, (i, h)
