@@ -287,7 +287,16 @@ struct SegTable {
   const int32_t* order;  // output pass: segments longest first (nullptr: in index order)
   int nseq, seq_len, L;
   int balance;  // the output pass evens its segments out over the heads' warm-ups (plan_segments)
-  int walk;  // pairs without warm-ups walk their whole sequence in one workgroup (no summary pass): walk_pays()
+  int walk;  // short sequences: every segment warms up as far back as it takes, no summary pass (seg_choice)
+  // States updated in place: copies of the initial states of the sequences of several segments (nullptr: none).
+  // Any segment may start from its sequence's initial state, and the last one writes the final state at a time
+  // that no launch order bounds; a sequence's copy is [Hv, D, D] fp32 at first_chunk / keep_len (one per
+  // sequence, since several segments are at least keep_len chunks).
+  float* kept;
+  int keep_len;
+  __device__ __forceinline__ float* kept_state(int s, int h, int Hv) const {
+    return kept + ((int64_t)(first_chunk(s) / keep_len) * Hv + h) * pf::D * pf::D;
+  }
   __device__ __forceinline__ int nch(int s) const {
     return cu ? chunk0[s + 1] - chunk0[s] : (seq_len + pf::CH - 1) / pf::CH;
   }
@@ -521,6 +530,23 @@ struct CaptureArgs {
   const int32_t* rows;
   int n_rows, C, K;
 };
+// The copies of states updated in place (SegTable::kept) as further workgroups, one per (sequence, value head).
+struct KeepArgs {
+  int n;  // workgroups (a multiple of 8; 0: no copies)
+  const float* states;
+  const int32_t* rows;
+  int n_rows;
+};
+__device__ void keep_one(int item, const KeepArgs& keep, const SegTable& tab, int Hv) {
+  const int s = item / Hv, h = item % Hv;
+  if (s >= tab.nseq || tab.nch(s) <= tab.L) return;
+  const int r0 = state_row(keep.rows, keep.n_rows, s);
+  if (r0 < 0) return;
+  const f32x4* src = reinterpret_cast<const f32x4*>(keep.states + ((int64_t)r0 * Hv + h) * pf::D * pf::D);
+  f32x4* dst = reinterpret_cast<f32x4*>(tab.kept_state(s, h, Hv));
+#pragma unroll 8
+  for (int i = threadIdx.x; i < pf::D * pf::D / 4; i += pf::NT) dst[i] = src[i];
+}
 
 // One wave per (chunk, value head) item (item = chunk slot * Hv + value head; a workgroup's 4 waves
 // are independent, so a wave past the end simply exits).  Lane (i, g) holds K[16 t + i][32 s + 8 g
@@ -535,11 +561,16 @@ __global__ __launch_bounds__(pf::NT, 2) void inv_kernel(const uint16_t* __restri
                                                        const int32_t* __restrict__ seq_chunk0, int nseq, int seq_len,
                                                        int64_t items, int Hqk, int Hv, int use_l2,
                                                        uint8_t* __restrict__ tfrag, float* __restrict__ knorm,
-                                                       SegTable tab, int* __restrict__ warm, CaptureArgs cap) {
+                                                       SegTable tab, int* __restrict__ warm, CaptureArgs cap, KeepArgs keep) {
   using namespace pf;
   if ((int)blockIdx.x < cap.n) {
     capture_one((int64_t)blockIdx.x * NT + threadIdx.x, cap.x, cap.x_stride, cap.rows_buf, cap.rows, cap.rows_buf,
                 cap.rows, cap.n_rows, cu, nseq, seq_len, cap.C, cap.K);
+    return;
+  }
+  const int extra = cap.n + keep.n;
+  if ((int)blockIdx.x < extra) {
+    keep_one((int)blockIdx.x - cap.n, keep, tab, Hv);
     return;
   }
   __shared__ float sdec[4][2][CH];                // per wave: G and beta by token
@@ -548,7 +579,7 @@ __global__ __launch_bounds__(pf::NT, 2) void inv_kernel(const uint16_t* __restri
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);  // the item is wave-uniform: scalar control flow
   // the 8 workgroups of one chunk's 32 value heads share an XCD, so the chunk's g and beta lines
   // (one token's heads per line) come from HBM once per chunk, not once per XCD
-  const int64_t item = xcd_range_item(blockIdx.x - cap.n, gridDim.x - cap.n) * 4 + w;
+  const int64_t item = xcd_range_item(blockIdx.x - extra, gridDim.x - extra) * 4 + w;
   if (item >= items) return;
   const int slot = (int)(item / Hv), h = (int)(item % Hv);
   const int r = Hv / Hqk, hk = h / r;
@@ -693,7 +724,7 @@ __global__ __launch_bounds__(pf::NT, 2) void inv_kernel(const uint16_t* __restri
     }
   // the last chunk of a segment with a successor: that transition slot's warm-up length
   const int nch = tab.nch(cp.seq);
-  if ((cp.c + 1) % tab.L == 0 && cp.c + 1 < nch) {
+  if (!tab.walk && (cp.c + 1) % tab.L == 0 && cp.c + 1 < nch) {
     const int ts = tab.first_slot(cp.seq) + (cp.c + 1) / tab.L - 1;
     const int wv = use_l2 ? chunk_warm(g, beta, Hv, h, cp.t0, tab.L) : 0;
     if (lane == 0) warm[(int64_t)ts * Hv + h] = wv;
@@ -1497,7 +1528,7 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
       s = tab.seq_of_seg(j);
       idx = j - tab.first_seg(s);
     }
-    if (idx > 0) slot = tab.first_slot(s) + idx - 1;  // the previous segment's slot holds this one's state
+    if (idx > 0 && !tab.walk) slot = tab.first_slot(s) + idx - 1;  // the previous segment's slot holds this one's state
     mode = kSegOut;
   } else {
     const int item = xcd_item(blockIdx.x, gridDim.x), rest = item >> 1;
@@ -1510,20 +1541,17 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
     mode = (item & 1) ? kSegA : kSegB;
     if (seq_warm_ok(tab, warm, Hv, h, s)) return;  // the output pass warms up instead
   }
-  const int nch_s = tab.nch(s), nseg_s = tab.nseg_of(nch_s);
-  const bool warm_ok = kPass == 0 && nseg_s > 1 && (slot >= 0 || tab.walk) && seq_warm_ok(tab, warm, Hv, h, s);
-  // a pair without warm-ups, short sequences: segment 0's workgroup runs all of it
-  const bool walk = kPass == 0 && tab.walk && nseg_s > 1 && !warm_ok;
-  if (walk && idx > 0) return;
-  const bool warm_path = slot >= 0 && warm_ok;
+  const int nch_s = tab.nch(s);
+  const bool warm_path = kPass == 0 && slot >= 0 && seq_warm_ok(tab, warm, Hv, h, s);
   // the output pass of a later segment on the exact path forms its initial state from the summaries of
   // the idx slots before it (ts_first .. ts_first + idx - 1)
   const int combine_steps = (kPass == 0 && slot >= 0 && !warm_path) ? idx : 0;
   const int ts_first = tab.first_slot(s);
   const int kh = h / (Hv / Hqk);
-  const bool even = plan.on && plan.end >= 0;  // a balanced segment: its own chunk range, warm-up or initial state
-  const int c_begin = even ? plan.begin : idx * tab.L;
-  const int n = even ? plan.end - plan.begin : walk || nch_s - c_begin < tab.L ? nch_s - c_begin : tab.L;
+  // a segment with a warm-up of its own (warm_before): a balanced one, or any of a short sequence
+  const bool even = kPass == 0 && (tab.walk || (plan.on && plan.end >= 0));
+  const int c_begin = plan.on && plan.end >= 0 ? plan.begin : idx * tab.L;
+  const int n = plan.on && plan.end >= 0 ? plan.end - plan.begin : nch_s - c_begin < tab.L ? nch_s - c_begin : tab.L;
   const int64_t t_seq = tab.start(s);
   const int Ls = tab.len(s);
   float* tslot = slot >= 0 ? trans + ((int64_t)slot * Hv + h) * sg::kTrans : nullptr;
@@ -1714,7 +1742,7 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
       const float* src = nullptr;
       if (mode == kSegOut && (even ? cb0 == 0 : slot < 0 || !warm_path) && init) {
         const int r0 = state_row(rows, n_rows, s);
-        if (r0 >= 0) src = init + ((int64_t)r0 * Hv + h) * D * D;
+        if (r0 >= 0) src = tab.kept && nch_s > tab.L ? tab.kept_state(s, h, Hv) : init + ((int64_t)r0 * Hv + h) * D * D;
       }
       if (src) {
 #pragma unroll
@@ -1819,7 +1847,7 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
     }
     // the state after the segment
     if (mode == kSegOut) {
-      if (final_state && (even ? c_begin + n == nch_s : walk || idx == nseg_s - 1)) {
+      if (final_state && c_begin + n == nch_s) {
         const int r0 = state_row(rows, n_rows, s);
         if (r0 >= 0) {
           float* dst = final_state + ((int64_t)r0 * Hv + h) * D * D;
@@ -2187,14 +2215,15 @@ int64_t seg_len(int64_t total_chunks, int nseq, int Hv) {
   return L < sg::kMinSeg ? sg::kMinSeg : L;
 }
 // Workspace layout: the segment table (nseq + 1 int32), the longest-first segment order (int32 per
-// segment), the transition flags (int32 per (slot,
+// segment, up to one per chunk), the transition flags (int32 per (slot,
 // value head)), the warm-up lengths (int32 per (slot, value head)), the transition slots (128 KiB per
-// (slot, value head): A's bf16 hi + lo fragments, then B in fp32; layout in namespace tr), the
+// (slot, value head): A's bf16 hi + lo fragments, then B in fp32; layout in namespace tr), the copies of
+// initial states updated in place (64 KiB per (slot, value head), SegTable::kept), the
 // inverse kernel's fragments (10 KiB per (chunk, value head): the bf16 hi half, then the lo half) and
 // its records of 64 K l2norm factors, the chunk's 64 g values and the lo flag (528 B per (chunk, value
 // head)), each part 256-byte aligned.
 struct SegLayout {
-  int64_t L, nslots, off_order, off_flags, off_warm, off_trans, off_tfrag, off_knorm, bytes;
+  int64_t L, nslots, off_order, off_flags, off_warm, off_trans, off_kept, off_tfrag, off_knorm, bytes;
 };
 SegLayout seg_layout(int64_t total_chunks, int nseq, int Hv) {
   auto up = [](int64_t x) { return (x + 255) / 256 * 256; };
@@ -2202,26 +2231,35 @@ SegLayout seg_layout(int64_t total_chunks, int nseq, int Hv) {
   l.L = seg_len(total_chunks, nseq, Hv);
   l.nslots = total_chunks / l.L;
   l.off_order = up(((int64_t)nseq + 1) * 4);
-  l.off_flags = l.off_order + up(((int64_t)nseq + total_chunks / l.L) * 4);  // segments: <= nseq + chunks / L
+  l.off_flags = l.off_order + up(((int64_t)nseq + total_chunks) * 4);  // segments: <= nseq + chunks
   l.off_warm = l.off_flags + up(l.nslots * Hv * 4);
   l.off_trans = l.off_warm + up(l.nslots * Hv * 4);
-  l.off_tfrag = l.off_trans + l.nslots * Hv * (int64_t)sg::kTrans * 4;
+  l.off_kept = l.off_trans + l.nslots * Hv * (int64_t)sg::kTrans * 4;
+  l.off_tfrag = l.off_kept + l.nslots * Hv * (int64_t)(pf::D * pf::D * 4);
   l.off_knorm = l.off_tfrag + total_chunks * Hv * (int64_t)tf::BYTES;
   l.bytes = l.off_knorm + total_chunks * Hv * (int64_t)(kr::FLOATS * 4);
   return l;
 }
-// Whether (sequence, value head) pairs without warm-ups walk their whole sequence in one workgroup instead
-// of taking the exact path; the call then needs no summary launch (2-3 us when every pair warms up).
-// In chunk steps of the walk (4.8 us each), the exact path costs about L for the outputs, 1.35 L per round
-// of 256 summary workgroups, and 0.75 per segment to combine: fitted on whole calls of 130 to 3000
-// tokens at 16, 32 and 48 value heads, e.g. slow decay, exact path against walk: 353 tokens x 48 heads
-// 54 / 48 us, 517 x 48 69 / 63, 700 x 48 78 / 73, 1000 x 48 93 / 97, 517 x 32 57 / 62, 517 x 16 54 / 60.
-// With the fused norm a step with outputs takes a third longer, the summaries' steps do not (the layer at
-// 517 tokens x 48 heads: 83.4 us on the exact path, 85.7 walked).
-bool walk_pays(int64_t max_seq_chunks, const SegLayout& lay, int Hv, bool norm) {
-  const int64_t segs = (max_seq_chunks + lay.L - 1) / lay.L, rounds = (2 * lay.nslots * Hv + 255) / 256;
-  const int64_t more = (27 * rounds * lay.L + 15 * (segs - 1)) * (norm ? 3 : 4) / 4;
-  return segs > 1 && 20 * max_seq_chunks <= 20 * lay.L + more;
+// The segments of a call.  Short sequences (walk) take no summary pass: every segment starts from a warm-up
+// as long as its head needs, at most from the sequence's start and its initial state, so a head of slow decay
+// costs its last segment one step per chunk of the sequence (3.9 us, most of them without outputs).  In such
+// steps the exact path costs about 1.25 L for the outputs, 1.65 L per round of 256 summary workgroups, and 0.9
+// per segment to combine: fitted on whole calls of 130 to 3000 tokens at 16, 32 and 48 value heads.  Slow
+// decay, exact path against walk: 353 tokens x 48 heads 54 / 42 us, 517 x 48 69 / 52, 700 x 48 78 / 60, 1000 x 48
+// 93 / 80, 517 x 32 58 / 52, 1000 x 32 82 / 80; fast decay, where the summary launch was 2-3 us for nothing,
+// 353 x 48 30 / 27.  Without summaries a segment may be a single chunk where the workgroups for it are free:
+// 353 x 32 at fast decay 27.4 us in 2-chunk segments, 22.2 in 1-chunk ones.
+struct SegChoice {
+  int L, walk;
+};
+SegChoice seg_choice(int64_t total_chunks, int nseq, int Hv, int seq_len, const SegLayout& lay) {
+  // A sequence spans several segments only beyond L chunks: seq_len is the uniform length, or for
+  // packed sequences an upper bound of the longest one (0: unknown)
+  const int64_t longest = seq_len > 0 ? ((int64_t)seq_len + pf::CH - 1) / pf::CH : total_chunks;
+  const int64_t segs = (longest + lay.L - 1) / lay.L, rounds = (2 * lay.nslots * Hv + 255) / 256;
+  if (segs <= 1 || 20 * longest > 25 * lay.L + 33 * rounds * lay.L + 18 * (segs - 1)) return {(int)lay.L, 0};
+  const bool one = lay.L == sg::kMinSeg && (total_chunks + nseq) * Hv <= sg::kTargetItems;
+  return {one ? 1 : (int)lay.L, 1};
 }
 }  // namespace
 
@@ -2284,32 +2322,33 @@ int chunk_prefill_impl(const void* q, int64_t q_stride, const void* k, int64_t k
   float* trans = (float*)(work + lay.off_trans);
   uint8_t* tfrag = work + lay.off_tfrag;
   float* knorm = (float*)(work + lay.off_knorm);
-  const int64_t nseg_max = (int64_t)nseq + total_chunks / lay.L;
+  const int64_t max_seq_chunks = seq_len > 0 ? ((int64_t)seq_len + pf::CH - 1) / pf::CH : total_chunks;
+  const SegChoice seg = seg_choice(total_chunks, nseq, Hv, seq_len, lay);
+  const int64_t nseg_max = (int64_t)nseq + total_chunks / seg.L;
   if (cu_seqlens && !table_built) {
-    seg_table_kernel<<<1, 256, 0, st>>>(seq_chunk0, nseq, (int)lay.L, seg0, order);
+    seg_table_kernel<<<1, 256, 0, st>>>(seq_chunk0, nseq, seg.L, seg0, order);
     int rc = check_launch("gdn_chunk_prefill(table)");
     if (rc) return rc;
   }
-  // A sequence spans several segments only beyond L chunks: seq_len is the uniform length, or for
-  // packed sequences an upper bound of the longest one (0: unknown)
-  const int64_t max_seq_chunks = seq_len > 0 ? ((int64_t)seq_len + pf::CH - 1) / pf::CH : total_chunks;
-  const int walk = walk_pays(max_seq_chunks, lay, Hv, norm_mode != 0) ? 1 : 0;
+  const bool in_place = initial_state && initial_state == final_state && max_seq_chunks > seg.L;
   // segments evened out over the heads' warm-ups: where one round of workgroups holds them all and a segment is
   // long enough for the heads to differ by more than the planning costs
-  const int balance = !walk && max_seq_chunks > lay.L && lay.L >= kBalanceMin && (int64_t)nseq * Hv <= sg::kTargetItems;
+  const int balance = !seg.walk && max_seq_chunks > lay.L && lay.L >= kBalanceMin && (int64_t)nseq * Hv <= sg::kTargetItems;
   const SegTable tab{cu_seqlens, seq_chunk0, cu_seqlens ? seg0 : nullptr, cu_seqlens ? order : nullptr, nseq, seq_len,
-                     (int)lay.L, balance, walk};
+                     seg.L, balance, seg.walk, in_place ? (float*)(work + lay.off_kept) : nullptr, (int)lay.L};
+  KeepArgs keep{};
+  if (in_place) keep = KeepArgs{(nseq * Hv + 7) / 8 * 8, initial_state, state_rows, n_rows};
   if (total_chunks > 0) {  // the intra-chunk inverses, one wave per (chunk, value head)
     const int64_t items = total_chunks * Hv;
-    const unsigned gi = (unsigned)((items + 3) / 4 + cap.n);
+    const unsigned gi = (unsigned)((items + 3) / 4 + cap.n + keep.n);
     if (beta_dtype == GDN_BF16)
       inv_kernel<uint16_t><<<gi, pf::NT, 0, st>>>((const uint16_t*)k, k_stride, g,
                                                   (const uint16_t*)beta, cu_seqlens, seq_chunk0, nseq, seq_len, items,
-                                                  Hqk, Hv, use_qk_l2norm, tfrag, knorm, tab, warm, cap);
+                                                  Hqk, Hv, use_qk_l2norm, tfrag, knorm, tab, warm, cap, keep);
     else
       inv_kernel<float><<<gi, pf::NT, 0, st>>>((const uint16_t*)k, k_stride, g,
                                                (const float*)beta, cu_seqlens, seq_chunk0, nseq, seq_len, items, Hqk,
-                                               Hv, use_qk_l2norm, tfrag, knorm, tab, warm, cap);
+                                               Hv, use_qk_l2norm, tfrag, knorm, tab, warm, cap, keep);
     int rc = check_launch("gdn_chunk_prefill(inverse)");
     if (rc) return rc;
   }
@@ -2326,7 +2365,7 @@ int chunk_prefill_impl(const void* q, int64_t q_stride, const void* k, int64_t k
     else GDN_SEG_LAUNCH(float);
 #undef GDN_SEG_LAUNCH
   };
-  if (!walk && lay.nslots > 0 && max_seq_chunks > lay.L) {  // segment summaries and their combination where no warm-up fits
+  if (!seg.walk && lay.nslots > 0 && max_seq_chunks > lay.L) {  // segment summaries and their combination where no warm-up fits
     launch(1, lay.nslots * Hv * 2);
     int rc = check_launch("gdn_chunk_prefill(summary)");
     if (rc) return rc;
@@ -2473,7 +2512,7 @@ extern "C" int gdn_chunk_prefill_inverse(const void* k, int64_t k_stride, const 
     const int rc = check_launch("gdn_chunk_prefill_inverse(table)");
     if (rc) return rc;
   }
-  const SegTable tab{cu_seqlens, seq_chunk0, cu_seqlens ? seg0 : nullptr, nullptr, nseq, seq_len, (int)lay.L, 0, 0};
+  const SegTable tab{cu_seqlens, seq_chunk0, cu_seqlens ? seg0 : nullptr, nullptr, nseq, seq_len, (int)lay.L, 0, 0, nullptr, 1};
   uint8_t* tfrag = work + lay.off_tfrag;
   float* knorm = (float*)(work + lay.off_knorm);
   int* warm = (int*)(work + lay.off_warm);
@@ -2482,11 +2521,11 @@ extern "C" int gdn_chunk_prefill_inverse(const void* k, int64_t k_stride, const 
   if (beta_dtype == GDN_BF16)
     inv_kernel<uint16_t><<<gi, pf::NT, 0, st>>>((const uint16_t*)k, k_stride, g, (const uint16_t*)beta, cu_seqlens,
                                                 seq_chunk0, nseq, seq_len, items, Hqk, Hv, use_qk_l2norm, tfrag,
-                                                knorm, tab, warm, CaptureArgs{});
+                                                knorm, tab, warm, CaptureArgs{}, KeepArgs{});
   else
     inv_kernel<float><<<gi, pf::NT, 0, st>>>((const uint16_t*)k, k_stride, g, (const float*)beta, cu_seqlens,
                                              seq_chunk0, nseq, seq_len, items, Hqk, Hv, use_qk_l2norm, tfrag, knorm,
-                                             tab, warm, CaptureArgs{});
+                                             tab, warm, CaptureArgs{}, KeepArgs{});
   int rc = check_launch("gdn_chunk_prefill_inverse(inverse)");
   if (rc) return rc;
   inv_records_expand_kernel<<<gi, 256, 0, st>>>(tfrag, knorm, items, t_out, use_qk_l2norm ? factor_out : nullptr);
@@ -2646,6 +2685,7 @@ extern "C" int gdn_prefill_layer_rows(const void* mixed, int64_t mixed_stride, c
   // state rows) the conv state capture
   const bool cap_fused = !conv_history || conv_history != conv_state;
   const SegLayout seg = seg_layout(total_chunks, nseq, Hv);
+  const SegChoice choice = seg_choice(total_chunks, nseq, Hv, seq_len, seg);
   PrologueArgs P{};
   P.x = (const uint16_t*)mixed;
   P.x_stride = mixed_stride;
@@ -2674,7 +2714,7 @@ extern "C" int gdn_prefill_layer_rows(const void* mixed, int64_t mixed_stride, c
   P.Hv = Hv;
   P.n_gate = (total_tokens * Hv + 255) / 256;
   P.chunk0 = seq_chunk0;
-  P.L = (int)seg.L;
+  P.L = choice.L;
   P.seg0 = (int32_t*)chunk_ws;
   P.order = (int32_t*)(chunk_ws + seg.off_order);
   P.table = cu_seqlens ? 1 : 0;

@@ -466,12 +466,14 @@ def test_gating(gdn, oracle, dev):
 
 
 
-@pytest.mark.parametrize("lens,n_rows", [([384], 1), ([385], 1), ([100, 0, 384, 65, 1], 7), ([700, 64, 353], 3)])
-def test_chunk_prefill_short_sequences_walk(gdn, oracle, dev, lens, n_rows):
-    """Short sequences: heads without a warm-up are walked from the start by their first segment's workgroup (384
-    tokens, 6 chunks, at these sizes; 385 tokens already take the summaries, as 700 do), while the other heads of
-    the call warm up.  Initial and final states in slot rows, in place; every (sequence, head) against the oracle."""
-    Hk, Hv, T = 2, 4, sum(lens)
+@pytest.mark.parametrize("lens,n_rows,Hk,Hv", [([576], 1, 2, 4), ([577], 1, 2, 4), ([100, 0, 576, 65, 1], 7, 2, 4),
+                                               ([700, 64, 353], 3, 2, 4), ([353], 2, 16, 48), ([517, 130], 3, 16, 32)])
+def test_chunk_prefill_short_sequences_walk(gdn, oracle, dev, lens, n_rows, Hk, Hv):
+    """Short sequences: every segment (of one chunk where the workgroups suffice, else of two or more) warms up as far
+    back as its head needs, to the sequence's start and its initial state for the heads of slow or no decay (576
+    tokens, 9 chunks, at 4 value heads; 577 tokens take the summaries there, as 700 do).  Initial and final states
+    in slot rows, in place; every (sequence, head) against the oracle."""
+    T, r = sum(lens), Hv // Hk
     q, k, v, g, beta, _ = _gdn_inputs(T, Hk, Hv, seed=T, state=False)
     g[..., 0] *= 10.0
     g[..., 1] *= 0.01
@@ -481,7 +483,7 @@ def test_chunk_prefill_short_sequences_walk(gdn, oracle, dev, lens, n_rows):
         cu.append(cu[-1] + n)
     slots = 0.02 * torch.randn(n_rows, Hv, 128, 128, generator=torch.Generator().manual_seed(5))
     rows = list(range(n_rows))[::-1][:len(lens)]
-    o_ref, s_ref = oracle.chunk_gated_delta_rule_varlen(_rep(q, 2), _rep(k, 2), v, g, beta, torch.tensor(cu), 64,
+    o_ref, s_ref = oracle.chunk_gated_delta_rule_varlen(_rep(q, r), _rep(k, r), v, g, beta, torch.tensor(cu), 64,
                                                         slots[rows], True, True)
     sd = slots.to(dev)
     o, _ = gdn.chunk_gated_delta_rule(q.to(dev), k.to(dev), v.to(dev), g.to(dev), beta.to(dev), initial_state=sd,
@@ -495,6 +497,33 @@ def test_chunk_prefill_short_sequences_walk(gdn, oracle, dev, lens, n_rows):
             assert rel_l2(sd[rows[i], h], s_ref[i, h]) <= STATE_TOL, (i, h)
     for spare in set(range(n_rows)) - set(rows):
         assert torch.equal(sd[spare].cpu(), slots[spare])
+
+
+@pytest.mark.parametrize("lens,Hk,Hv,scale", [([353] * 9, 16, 48, 0.01), ([353, 100, 700] * 3, 16, 48, 1.0),
+                                              ([2000, 0, 1500, 64] * 3, 16, 32, 0.01), ([16447], 16, 32, 0.3)])
+def test_chunk_prefill_states_in_place_match_separate_buffers(gdn, dev, lens, Hk, Hv, scale):
+    """More segments than the chip runs at once, states updated in their slot rows: every segment that starts from
+    its sequence's initial state finds it whole, also when the last segment has already written the row.  The same
+    bits as with separate initial and final buffers, the rows of empty sequences and spare rows included."""
+    T = sum(lens)
+    q, k, v, g, beta, _ = (x.to(dev) if x is not None else None for x in _gdn_inputs(T, Hk, Hv, seed=T, state=False))
+    g *= scale
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    n_rows = len(lens) + 1
+    rows = list(range(n_rows))[::-1][:len(lens)]
+    slots = 0.02 * torch.randn(n_rows, Hv, 128, 128, generator=torch.Generator().manual_seed(6)).to(dev)
+
+    def run(init, final):
+        return gdn.chunk_gated_delta_rule(q, k, v, g, beta, initial_state=init, cu_seqlens=cu, state_rows=rows,
+                                          final_state_out=final, use_qk_l2norm_in_kernel=True)[0]
+
+    separate, inplace = slots.clone(), slots.clone()
+    o_sep = run(slots, separate)
+    o_in = run(inplace, inplace)
+    assert torch.equal(o_in, o_sep)
+    assert torch.equal(inplace, separate)
 
 
 @pytest.mark.parametrize("lens,Hk,Hv,exact", [([16447], 16, 32, False), ([20000, 9000, 0, 3000], 8, 16, True),
