@@ -14,8 +14,8 @@
 // consecutive chunks and walks
 // one segment per workgroup with the fp32 state in MFMA accumulators, building every other operand
 // of a chunk in LDS (local waves) while the chain waves run the previous chunk.  A segment's true
-// initial state comes from a warm-up over the end of the segment before it, or from a summary
-// pass plus an fp32 combination.  Products run on v_mfma_f32_16x16x32_bf16 with fp32
+// initial state comes from a warm-up over the chunks before it (in short sequences as far back as
+// their start), or from a summary pass plus an fp32 combination.  Products run on v_mfma_f32_16x16x32_bf16 with fp32
 // accumulation; the state update feeds DEC vn as a bf16 hi + lo pair, so the running state never
 // sees a bf16 rounding of its increment.
 #include "gdn_device.h"
@@ -246,7 +246,8 @@ namespace sg {
 constexpr int NT = 512;                      // 8 waves
 // Shortest segment the host cuts (chunks).  2: a short prompt's heads spread over more workgroups
 // (353 tokens at 48 value heads: segments of 2 chunks, 3 chunk steps a workgroup instead of 5);
-// a later segment's warm-up must then fit in the 2 chunks before it.
+// where the call takes summaries, a later segment's warm-up must then fit in the 2 chunks before it.
+// (Short sequences take none, and single-chunk segments where workgroups are free: seg_choice.)
 constexpr int kMinSeg = 2;
 constexpr int kTargetItems = 256;            // segments x value heads the host aims for
 constexpr float kNegligibleLog = -44.3614f;  // ln(2^-64): a segment map A_j this small is not formed
@@ -563,14 +564,13 @@ __global__ __launch_bounds__(pf::NT, 2) void inv_kernel(const uint16_t* __restri
                                                        uint8_t* __restrict__ tfrag, float* __restrict__ knorm,
                                                        SegTable tab, int* __restrict__ warm, CaptureArgs cap, KeepArgs keep) {
   using namespace pf;
-  if ((int)blockIdx.x < cap.n) {
-    capture_one((int64_t)blockIdx.x * NT + threadIdx.x, cap.x, cap.x_stride, cap.rows_buf, cap.rows, cap.rows_buf,
-                cap.rows, cap.n_rows, cu, nseq, seq_len, cap.C, cap.K);
-    return;
-  }
   const int extra = cap.n + keep.n;
   if ((int)blockIdx.x < extra) {
-    keep_one((int)blockIdx.x - cap.n, keep, tab, Hv);
+    if ((int)blockIdx.x < cap.n)
+      capture_one((int64_t)blockIdx.x * NT + threadIdx.x, cap.x, cap.x_stride, cap.rows_buf, cap.rows, cap.rows_buf,
+                  cap.rows, cap.n_rows, cu, nseq, seq_len, cap.C, cap.K);
+    else
+      keep_one((int)blockIdx.x - cap.n, keep, tab, Hv);
     return;
   }
   __shared__ float sdec[4][2][CH];                // per wave: G and beta by token
@@ -1489,8 +1489,8 @@ __device__ __forceinline__ void chain_part2(const SegBuf& B, ChainRegs& R, int l
 }
 
 // Segment kernel.  pass 0 (output): one workgroup per (segment, value head) from the segment's
-// initial state (the sequence's initial state row, zero, or the combined state of the previous
-// segment in its transition slot), writing o and, at a sequence's last segment, the final state.
+// initial state (the sequence's initial state, zero before a warm-up, or the combination of the
+// summaries in the slots before it), writing o and, at a sequence's last segment, the final state.
 // pass 1 (summary): two workgroups per (transition slot, value head): B (from zero, with U) and A
 // (from the identity, without U), written into the slot; A is skipped when negligible.
 // Waves 0-3 (local) prepare chunk c+1's operands in one buffer (and store chunk c-1's outputs) while
