@@ -2244,9 +2244,11 @@ SegLayout seg_layout(int64_t total_chunks, int nseq, int Hv) {
 // as long as its head needs, at most from the sequence's start and its initial state, so a head of slow decay
 // costs its last segment one step per chunk of the sequence (3.9 us, most of them without outputs).  In such
 // steps the exact path costs about 1.25 L for the outputs, 1.65 L per round of 256 summary workgroups, and 0.9
-// per segment to combine: fitted on whole calls of 130 to 3000 tokens at 16, 32 and 48 value heads.  Slow
-// decay, exact path against walk: 353 tokens x 48 heads 54 / 42 us, 517 x 48 69 / 52, 700 x 48 78 / 60, 1000 x 48
-// 93 / 80, 517 x 32 58 / 52, 1000 x 32 82 / 80; fast decay, where the summary launch was 2-3 us for nothing,
+// per segment to combine: fitted on whole calls of 130 to 3000 tokens at 16, 32 and 48 value heads.  The rule
+// counts one round, as where only a few heads are slow (the host cannot know): 1000 tokens x 48 heads, two rounds
+// when every head is slow, walk 80 us against 93 then, but 92 against 89 in the layer with a few slow heads, and
+// so take the exact path.  Slow decay, exact path against walk: 353 tokens x 48 heads 54 / 42 us, 517 x 48 69 / 52,
+// 700 x 48 78 / 60, 517 x 32 58 / 52; fast decay, where the summary launch was 2-3 us for nothing,
 // 353 x 48 30 / 27.  Without summaries a segment may be a single chunk where the workgroups for it are free:
 // 353 x 32 at fast decay 27.4 us in 2-chunk segments, 22.2 in 1-chunk ones.
 struct SegChoice {
@@ -2256,8 +2258,8 @@ SegChoice seg_choice(int64_t total_chunks, int nseq, int Hv, int seq_len, const 
   // A sequence spans several segments only beyond L chunks: seq_len is the uniform length, or for
   // packed sequences an upper bound of the longest one (0: unknown)
   const int64_t longest = seq_len > 0 ? ((int64_t)seq_len + pf::CH - 1) / pf::CH : total_chunks;
-  const int64_t segs = (longest + lay.L - 1) / lay.L, rounds = (2 * lay.nslots * Hv + 255) / 256;
-  if (segs <= 1 || 20 * longest > 25 * lay.L + 33 * rounds * lay.L + 18 * (segs - 1)) return {(int)lay.L, 0};
+  const int64_t segs = (longest + lay.L - 1) / lay.L;
+  if (segs <= 1 || 20 * longest > 58 * lay.L + 18 * (segs - 1)) return {(int)lay.L, 0};
   const bool one = lay.L == sg::kMinSeg && (total_chunks + nseq) * Hv <= sg::kTargetItems;
   return {one ? 1 : (int)lay.L, 1};
 }
