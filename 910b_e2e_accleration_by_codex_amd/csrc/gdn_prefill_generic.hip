@@ -340,6 +340,8 @@ struct GenWindow {
   float* carry;  // states between windows [ns, Hv, Dk, Dv], or null with one window
   int s0, ns;    // the group's sequences s0 .. s0 + ns - 1
   int c0, nw;    // the window's chunks c0 .. c0 + nw - 1
+  int maxch;     // chunks of the longest sequence as the caller bounds it: no sequence runs past it (the carry
+                 // exists for the windows that this bound makes, whatever the device table says)
 };
 
 template <int DK>
@@ -597,7 +599,7 @@ __global__ __launch_bounds__(512) void generic_chain_kernel(GenArgs P, GenWindow
   const int h = rest % P.Hv, s = W.s0 + rest / P.Hv;
   const int64_t t_seq = P.cu ? (int64_t)P.cu[s] : (int64_t)s * P.seq_len;
   const int Ls = P.cu ? P.cu[s + 1] - P.cu[s] : P.seq_len;
-  const int nch = (Ls + CH - 1) / CH;
+  const int nch_s = (Ls + CH - 1) / CH, nch = nch_s < W.maxch ? nch_s : W.maxch;
   const int cnt = nch - W.c0 < W.nw ? nch - W.c0 : W.nw;  // chunks of this window
   if (W.c0 > 0 && cnt <= 0) return;                       // the sequence ended in an earlier window
   const int64_t istride = (int64_t)P.Hv * item_floats(DK, P.Dv);
@@ -744,7 +746,7 @@ static void launch_generic_ws(const GenArgs& P, const gp::Plan& pl, float* work,
     int c0 = 0;
     do {  // (no chunks at all: the chain alone hands the initial states on)
       const int nw = pl.maxch - c0 < pl.nw ? pl.maxch - c0 : pl.nw;
-      const GenWindow W{work, carry, s0, ns, c0, nw < 1 ? 1 : nw};
+      const GenWindow W{work, carry, s0, ns, c0, nw < 1 ? 1 : nw, pl.maxch};
       if (nw > 0) generic_prep_kernel<DK, DT><<<(unsigned)((int64_t)ns * nw * P.Hv), kPrepThreads, 0, st>>>(P, W);
       generic_chain_kernel<DK, DT><<<(unsigned)((int64_t)ns * P.Hv * (P.Dv / 16)), 512, 0, st>>>(P, W);
       c0 += pl.nw;
@@ -828,6 +830,9 @@ extern "C" int gdn_chunk_prefill_generic_ws(const void* q, int64_t q_stride, con
                                beta_dtype, state_rows, n_rows, out, total_tokens, cu_seqlens, nseq, seq_len, Hqk, Hv,
                                Dk, Dv, in_dtype);
   if (rc) return rc;
+  GDN_REQUIRE((int64_t)nseq * seq_len >= total_tokens,
+              "gdn_chunk_prefill_generic_ws: seq_len %d cannot bound %d sequences of %lld tokens", seq_len, nseq,
+              (long long)total_tokens);
   if (nseq == 0) return GDN_OK;
   const gp::Plan pl = gp::plan(nseq, seq_len, Hv, Dk, Dv);
   GDN_REQUIRE(workspace && aligned(workspace, 16) && workspace_bytes >= pl.bytes,

@@ -156,8 +156,10 @@ int gdn_chunk_prefill_generic(const void* q, int64_t q_stride, const void* k, in
  * gdn_chunk_prefill_generic with a workspace: the same rule, in fp32 throughout, in two kernels -- the
  * state-independent part of every chunk in parallel, then the state chain over 16 value columns per
  * workgroup.  Arguments as gdn_chunk_prefill_generic, except that with cu_seqlens seq_len must be an
- * upper bound of every sequence's length (a bound below a sequence's true length drops that
- * sequence's later chunks), and out must be 16-byte aligned.
+ * upper bound of every sequence's length (one that cannot hold total_tokens, nseq seq_len < total_tokens,
+ * 0 included, is refused with GDN_EINVAL; one below a sequence's true length drops that sequence's
+ * chunks past it: their outputs are not written and the final state is the one before them), and out must
+ * be 16-byte aligned.
  *   workspace: 16-byte aligned, gdn_chunk_prefill_generic_workspace_bytes(nseq, seq_len, Hv, Dk, Dv)
  *     bytes (-1 for bad sizes): about (3 Dk + Dv + 40) * 256 bytes per (chunk, value head), capped near
  *     256 MiB (longer calls run in windows of chunks, several launches each); contents are scratch.

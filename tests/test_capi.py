@@ -100,6 +100,11 @@ def test_version_limits_and_error_path(lib):
     rc = h.gdn_chunk_prefill_generic(p, 256, p, 256, p, 256, p, p, 0, None, None, None, 1, p, 65, None, 1, 64, 2,
                                      2, 64, 64, 0, 1, None)
     assert rc == 1 and b"nseq*seq_len" in h.gdn_last_error()
+    # with a workspace: a bound that cannot hold the packed tokens (0 included) is refused before any launch
+    for bound in (0, 31):
+        rc = h.gdn_chunk_prefill_generic_ws(p, 128, p, 128, p, 128, p, p, 0, None, p, None, 2, p, 64, p, 2, bound, 2,
+                                            2, 64, 64, 0, 1, p, 1 << 30, None)
+        assert rc == 1 and b"seq_len" in h.gdn_last_error()
     # gdn_chunk_prefill hands other dtypes and head dims to the generic rule (whose checks then run)
     rc = h.gdn_chunk_prefill(p, 0, p, 0, p, 0, p, p, 1, None, None, p, 64, None, None, 1, 1, 64, 16, 32, 96, 0, 1,
                              p, 1 << 30, None)

@@ -232,3 +232,37 @@ def test_generic_windows_and_groups_match_the_workspace_free_kernel(gdn, oracle,
         assert rel_l2(s[i], s_ref[0]) <= (FP32_TOL if dtype == torch.float32 else 1e-3)
         if lens[i]:
             assert rel_l2(o[:, sl].float(), o_ref.float()) <= (FP32_TOL if dtype == torch.float32 else 1e-2)
+
+
+@pytest.mark.parametrize("Dk,Dv", [(64, 64), (128, 32)])
+def test_generic_short_length_bound_stays_in_the_workspace(gdn, dev, Dk, Dv):
+    """A seq_len one chunk below a sequence's true length (130 tokens, bound 128): that sequence's last chunk is
+    dropped -- its outputs stay as they were, its final state is the one before it -- and nothing is written past
+    the workspace; the other sequences are whole.  Bit for bit the call on the sequences cut at the bound."""
+    from importlib import import_module
+    lib = import_module(gdn.__name__ + "._lib")
+    H, lens, bound, guard = 2, [130, 64, 64], 128, 1 << 20
+    cu, T = [0, 130, 194, 258], 258
+    r = torch.Generator().manual_seed(17)
+    q, k, v = (torch.randn(T, H, d, generator=r).to(dev) for d in (Dk, Dk, Dv))
+    beta, g = torch.rand(T, H, generator=r).to(dev), -0.1 * torch.rand(T, H, generator=r).to(dev)
+    s0 = 0.1 * torch.randn(len(lens), H, Dk, Dv, generator=r).to(dev)
+    p = lib.ptr
+
+    def run(q, k, v, g, beta, cu):
+        table, n = torch.tensor(cu, dtype=torch.int32).to(dev), q.shape[0]
+        need = int(lib.lib().gdn_chunk_prefill_generic_workspace_bytes(len(lens), bound, H, Dk, Dv))
+        work = torch.full((need + guard,), 0x5A, dtype=torch.uint8, device=dev)
+        out, fin = torch.full((n, H, Dv), 7.0, device=dev), torch.empty_like(s0)
+        lib.call("gdn_chunk_prefill_generic_ws", p(q), q.stride(0), p(k), k.stride(0), p(v), v.stride(0), p(g), p(beta),
+                 lib.F32, p(s0), p(fin), None, len(lens), p(out), n, p(table), len(lens), bound, H, H, Dk, Dv, lib.F32, 1,
+                 p(work), need, lib.stream_of(q))
+        torch.cuda.synchronize()
+        assert bool((work[need:] == 0x5A).all())
+        return out, fin
+
+    out, fin = run(q, k, v, g, beta, cu)
+    keep = [i for i in range(T) if not 128 <= i < 130]
+    cut_out, cut_fin = run(*(x[keep].contiguous() for x in (q, k, v, g, beta)), [0, 128, 192, 256])
+    assert bool((out[128:130] == 7.0).all())
+    assert torch.equal(out[keep], cut_out) and torch.equal(fin, cut_fin)
