@@ -287,17 +287,6 @@ struct SegTable {
   const int32_t* seg0;
   const int32_t* order;  // output pass: segments longest first (nullptr: in index order)
   int nseq, seq_len, L;
-  int balance;  // the output pass evens its segments out over the heads' warm-ups (plan_segments)
-  int walk;  // short sequences: every segment warms up as far back as it takes, no summary pass (seg_choice)
-  // States updated in place: copies of the initial states of the sequences of several segments (nullptr: none).
-  // Any segment may start from its sequence's initial state, and the last one writes the final state at a time
-  // that no launch order bounds; a sequence's copy is [Hv, D, D] fp32 at first_chunk / keep_len (one per
-  // sequence, since several segments are at least keep_len chunks).
-  float* kept;
-  int keep_len;
-  __device__ __forceinline__ float* kept_state(int s, int h, int Hv) const {
-    return kept + ((int64_t)(first_chunk(s) / keep_len) * Hv + h) * pf::D * pf::D;
-  }
   __device__ __forceinline__ int nch(int s) const {
     return cu ? chunk0[s + 1] - chunk0[s] : (seq_len + pf::CH - 1) / pf::CH;
   }
@@ -331,6 +320,24 @@ struct SegTable {
     return lo;
   }
 };
+
+// What only the calls with segments of other forms need (kForm, kMore below); the others' kernels do not take it.
+struct SegOwn {
+  int balance;  // the output pass evens its segments out over the heads' warm-ups (plan_segments)
+  int walk;  // short sequences: every segment warms up as far back as it takes, no summary pass (seg_choice)
+  // States updated in place: copies of the initial states of the sequences of several segments (nullptr: none).
+  // Any segment may start from its sequence's initial state, and the last one writes the final state at a time
+  // that no launch order bounds; a sequence's copy is [Hv, D, D] fp32 at first_chunk / keep_len (one per
+  // sequence, since several segments are at least keep_len chunks).
+  float* kept;
+  int keep_len;
+  __device__ __forceinline__ float* kept_state(const SegTable& tab, int s, int h, int Hv) const {
+    return kept + ((int64_t)(tab.first_chunk(s) / keep_len) * Hv + h) * pf::D * pf::D;
+  }
+};
+struct NoArgs {};
+template <bool kOn, typename T>
+using ArgsIf = std::conditional_t<kOn, T, NoArgs>;
 
 // Inclusive scan of part[0..255] in place (all 256 threads; barriers inside).
 __device__ __forceinline__ void block_scan256(int* part, int t) {
@@ -538,40 +545,51 @@ struct KeepArgs {
   const int32_t* rows;
   int n_rows;
 };
-__device__ void keep_one(int item, const KeepArgs& keep, const SegTable& tab, int Hv) {
+__device__ void keep_one(int item, const KeepArgs& keep, const SegTable& tab, const SegOwn& own, int Hv) {
   const int s = item / Hv, h = item % Hv;
   if (s >= tab.nseq || tab.nch(s) <= tab.L) return;
   const int r0 = state_row(keep.rows, keep.n_rows, s);
   if (r0 < 0) return;
   const f32x4* src = reinterpret_cast<const f32x4*>(keep.states + ((int64_t)r0 * Hv + h) * pf::D * pf::D);
-  f32x4* dst = reinterpret_cast<f32x4*>(tab.kept_state(s, h, Hv));
+  f32x4* dst = reinterpret_cast<f32x4*>(own.kept_state(tab, s, h, Hv));
 #pragma unroll 8
   for (int i = threadIdx.x; i < pf::D * pf::D / 4; i += pf::NT) dst[i] = src[i];
 }
 
+struct InvMore {
+  SegOwn own;
+  CaptureArgs cap;
+  KeepArgs keep;
+};
 // One wave per (chunk, value head) item (item = chunk slot * Hv + value head; a workgroup's 4 waves
 // are independent, so a wave past the end simply exits).  Lane (i, g) holds K[16 t + i][32 s + 8 g
 // .. + 7] for token tiles t and k-blocks s < 4: the A fragment of tile t and, as K^T, the B
 // fragment of tile t, so K K^T needs nothing but these registers.  (Waves that each take several
 // items and prefetch the next one's inputs need more registers, halve the resident waves and were
 // measured slower.)
-template <typename BetaT>
+// kMore: further workgroups (cap, keep) or segments with warm-ups of their own (the records' chunk sums); the
+// calls with none of them run a kernel without that code and its arguments, as the output pass does (kForm).
+template <typename BetaT, bool kMore>
 __global__ __launch_bounds__(pf::NT, 2) void inv_kernel(const uint16_t* __restrict__ k, int64_t ks,
                                                        const float* __restrict__ g, const BetaT* __restrict__ beta,
                                                        const int32_t* __restrict__ cu,
                                                        const int32_t* __restrict__ seq_chunk0, int nseq, int seq_len,
                                                        int64_t items, int Hqk, int Hv, int use_l2,
                                                        uint8_t* __restrict__ tfrag, float* __restrict__ knorm,
-                                                       SegTable tab, int* __restrict__ warm, CaptureArgs cap, KeepArgs keep) {
+                                                       SegTable tab, int* __restrict__ warm, ArgsIf<kMore, InvMore> more) {
   using namespace pf;
-  const int extra = cap.n + keep.n;
-  if ((int)blockIdx.x < extra) {
-    if ((int)blockIdx.x < cap.n)
-      capture_one((int64_t)blockIdx.x * NT + threadIdx.x, cap.x, cap.x_stride, cap.rows_buf, cap.rows, cap.rows_buf,
-                  cap.rows, cap.n_rows, cu, nseq, seq_len, cap.C, cap.K);
-    else
-      keep_one((int)blockIdx.x - cap.n, keep, tab, Hv);
-    return;
+  int extra = 0;
+  if constexpr (kMore) {
+    const CaptureArgs& cap = more.cap;
+    extra = cap.n + more.keep.n;
+    if ((int)blockIdx.x < extra) {
+      if ((int)blockIdx.x < cap.n)
+        capture_one((int64_t)blockIdx.x * NT + threadIdx.x, cap.x, cap.x_stride, cap.rows_buf, cap.rows, cap.rows_buf,
+                    cap.rows, cap.n_rows, cu, nseq, seq_len, cap.C, cap.K);
+      else
+        keep_one((int)blockIdx.x - cap.n, more.keep, tab, more.own, Hv);
+      return;
+    }
   }
   __shared__ float sdec[4][2][CH];                // per wave: G and beta by token
   __shared__ float strp[4][4 * 16 * kTrPitch];    // per wave: 4 transpose tiles
@@ -686,14 +704,12 @@ __global__ __launch_bounds__(pf::NT, 2) void inv_kernel(const uint16_t* __restri
   bool lo_rec = __expf(Gl) > sg::kPreciseGl || Gl > sg::kLoRecordLog;
   if (!lo_rec)
     lo_rec = tail_decay_above(g, Hv, h, t_tail, t_end, sg::kLoRecordLog, gtail);
-  {  // (a NaN in g makes the sum one)
+  if (lane == 0)
+    reinterpret_cast<int*>(knorm)[((int64_t)slot * Hv + h) * kr::FLOATS + kr::FLAG] = lo_rec ? 1 : 0;
+  if (kMore) {  // (a NaN in g makes the sum one)
     const float b = sdec[w][1][lane];
     const bool ok = use_l2 && __builtin_amdgcn_ballot_w64(!(b >= 0.f && b <= 1.f)) == 0;
-    if (lane == 0) {
-      float* rec = knorm + ((int64_t)slot * Hv + h) * kr::FLOATS;
-      reinterpret_cast<int*>(rec)[kr::FLAG] = lo_rec ? 1 : 0;
-      rec[kr::SUM] = ok ? Gl : __builtin_nanf("");
-    }
+    if (lane == 0) knorm[((int64_t)slot * Hv + h) * kr::FLOATS + kr::SUM] = ok ? Gl : __builtin_nanf("");
   }
   // fragments (w', s), s <= w' / 2: element e of lane (i, g) = T[16 w' + i][j] beta_j with
   // j = 32 s + kpos(8 g + e), kpos(8 g + e) = 16 (e >> 2) + 4 g + (e & 3): blocks 2s (e < 4) and 2s + 1
@@ -724,7 +740,9 @@ __global__ __launch_bounds__(pf::NT, 2) void inv_kernel(const uint16_t* __restri
     }
   // the last chunk of a segment with a successor: that transition slot's warm-up length
   const int nch = tab.nch(cp.seq);
-  if (!tab.walk && (cp.c + 1) % tab.L == 0 && cp.c + 1 < nch) {
+  bool walk = false;
+  if constexpr (kMore) walk = more.own.walk;
+  if (!walk && (cp.c + 1) % tab.L == 0 && cp.c + 1 < nch) {
     const int ts = tab.first_slot(cp.seq) + (cp.c + 1) / tab.L - 1;
     const int wv = use_l2 ? chunk_warm(g, beta, Hv, h, cp.t0, tab.L) : 0;
     if (lane == 0) warm[(int64_t)ts * Hv + h] = wv;
@@ -1495,12 +1513,18 @@ __device__ __forceinline__ void chain_part2(const SegBuf& B, ChainRegs& R, int l
 // (from the identity, without U), written into the slot; A is skipped when negligible.
 // Waves 0-3 (local) prepare chunk c+1's operands in one buffer (and store chunk c-1's outputs) while
 // waves 4-7 (chain) run chunk c from the other: two LDS barriers a chunk, met by both roles.
-template <typename BetaT, typename OutT, int kPass, int kNorm = 0>
+// kForm (pass 0): kFixed, segments of L chunks; kOwnWalk, those of short sequences (every segment warms up as far back
+// as it takes); kOwnEven, those evened out by plan_segments (own.balance).  States kept aside (own.kept) need one of
+// the last two.  Each form runs a kernel without the others' code and arguments: with all of it in one kernel, 16
+// fresh prompts of 8 to 64 tokens x 32 heads through the layer took 49.0-49.3 us against 48.0-48.7 (over several
+// builds: where the code comes to lie moves these calls by up to 0.5 us), 353 tokens x 48 heads 26.2 against 25.9.
+enum SegForm { kFixed = 0, kOwnWalk = 1, kOwnEven = 2 };
+template <typename BetaT, typename OutT, int kPass, int kNorm = 0, int kForm = kFixed>
 __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
     const uint16_t* __restrict__ q, int64_t qs, const uint16_t* __restrict__ k, int64_t ks, const uint16_t* __restrict__ v,
     int64_t vs, const float* __restrict__ g,
-    const BetaT* __restrict__ beta, OutT* __restrict__ out, SegTable tab, int Hqk, int Hv, int use_l2,
-    const float* __restrict__ init,
+    const BetaT* __restrict__ beta, OutT* __restrict__ out, SegTable tab, ArgsIf<kForm != kFixed, SegOwn> own, int Hqk, int Hv,
+    int use_l2, const float* __restrict__ init,
     const int32_t* __restrict__ rows, int n_rows, float* __restrict__ final_state, float* __restrict__ trans,
     int* __restrict__ tflags, const uint8_t* __restrict__ tfrag, const float* __restrict__ knorm,
     const int* __restrict__ warm, GateArgs gate) {
@@ -1512,10 +1536,13 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
   const int t = threadIdx.x, w = t >> 6, lane = t & 63, c16 = lane & 15, g4 = lane >> 4;
   int mode, h, s, idx, slot = -1;
   PlanItem plan{false, false, 0, 0, 0, 0};
+  constexpr bool walk = kForm == kOwnWalk;
   if (kPass == 0) {
     const int item = xcd_item(blockIdx.x, gridDim.x);
-    if (tab.balance) plan = plan_segments(reinterpret_cast<PlanSmem&>(sm), tab, warm, Hqk, Hv, item);
-    if (plan.on) {
+    if constexpr (kForm == kOwnEven) {
+      if (own.balance) plan = plan_segments(reinterpret_cast<PlanSmem&>(sm), tab, warm, Hqk, Hv, item);
+    }
+    if (kForm == kOwnEven && plan.on) {
       if (plan.idle) return;
       s = plan.s;
       h = plan.h;
@@ -1528,7 +1555,7 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
       s = tab.seq_of_seg(j);
       idx = j - tab.first_seg(s);
     }
-    if (idx > 0 && !tab.walk) slot = tab.first_slot(s) + idx - 1;  // the previous segment's slot holds this one's state
+    if (idx > 0 && !walk) slot = tab.first_slot(s) + idx - 1;  // the previous segment's slot holds this one's state
     mode = kSegOut;
   } else {
     const int item = xcd_item(blockIdx.x, gridDim.x), rest = item >> 1;
@@ -1549,9 +1576,10 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
   const int ts_first = tab.first_slot(s);
   const int kh = h / (Hv / Hqk);
   // a segment with a warm-up of its own (warm_before): a balanced one, or any of a short sequence
-  const bool even = kPass == 0 && (tab.walk || (plan.on && plan.end >= 0));
-  const int c_begin = plan.on && plan.end >= 0 ? plan.begin : idx * tab.L;
-  const int n = plan.on && plan.end >= 0 ? plan.end - plan.begin : nch_s - c_begin < tab.L ? nch_s - c_begin : tab.L;
+  const bool planned = kForm == kOwnEven && plan.on && plan.end >= 0;
+  const bool even = walk || planned;
+  const int c_begin = planned ? plan.begin : idx * tab.L;
+  const int n = planned ? plan.end - plan.begin : nch_s - c_begin < tab.L ? nch_s - c_begin : tab.L;
   const int64_t t_seq = tab.start(s);
   const int Ls = tab.len(s);
   float* tslot = slot >= 0 ? trans + ((int64_t)slot * Hv + h) * sg::kTrans : nullptr;
@@ -1742,7 +1770,9 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
       const float* src = nullptr;
       if (mode == kSegOut && (even ? cb0 == 0 : slot < 0 || !warm_path) && init) {
         const int r0 = state_row(rows, n_rows, s);
-        if (r0 >= 0) src = tab.kept && nch_s > tab.L ? tab.kept_state(s, h, Hv) : init + ((int64_t)r0 * Hv + h) * D * D;
+        if (r0 >= 0) src = init + ((int64_t)r0 * Hv + h) * D * D;
+        if constexpr (kForm != kFixed)
+          if (r0 >= 0 && own.kept && nch_s > tab.L) src = own.kept_state(tab, s, h, Hv);
       }
       if (src) {
 #pragma unroll
@@ -2337,35 +2367,54 @@ int chunk_prefill_impl(const void* q, int64_t q_stride, const void* k, int64_t k
   // long enough for the heads to differ by more than the planning costs
   const int balance = !seg.walk && max_seq_chunks > lay.L && lay.L >= kBalanceMin && (int64_t)nseq * Hv <= sg::kTargetItems;
   const SegTable tab{cu_seqlens, seq_chunk0, cu_seqlens ? seg0 : nullptr, cu_seqlens ? order : nullptr, nseq, seq_len,
-                     seg.L, balance, seg.walk, in_place ? (float*)(work + lay.off_kept) : nullptr, (int)lay.L};
+                     seg.L};
+  const SegOwn own{balance, seg.walk, in_place ? (float*)(work + lay.off_kept) : nullptr, (int)lay.L};
+  const bool use_own = seg.walk || balance || in_place;
   KeepArgs keep{};
   if (in_place) keep = KeepArgs{(nseq * Hv + 7) / 8 * 8, initial_state, state_rows, n_rows};
   if (total_chunks > 0) {  // the intra-chunk inverses, one wave per (chunk, value head)
     const int64_t items = total_chunks * Hv;
     const unsigned gi = (unsigned)((items + 3) / 4 + cap.n + keep.n);
-    if (beta_dtype == GDN_BF16)
-      inv_kernel<uint16_t><<<gi, pf::NT, 0, st>>>((const uint16_t*)k, k_stride, g,
-                                                  (const uint16_t*)beta, cu_seqlens, seq_chunk0, nseq, seq_len, items,
-                                                  Hqk, Hv, use_qk_l2norm, tfrag, knorm, tab, warm, cap, keep);
-    else
-      inv_kernel<float><<<gi, pf::NT, 0, st>>>((const uint16_t*)k, k_stride, g,
-                                               (const float*)beta, cu_seqlens, seq_chunk0, nseq, seq_len, items, Hqk,
-                                               Hv, use_qk_l2norm, tfrag, knorm, tab, warm, cap, keep);
+#define GDN_INV_LAUNCH(BT, MORE, ...)                                                                                \
+  inv_kernel<BT, MORE><<<gi, pf::NT, 0, st>>>((const uint16_t*)k, k_stride, g, (const BT*)beta, cu_seqlens, seq_chunk0, \
+                                              nseq, seq_len, items, Hqk, Hv, use_qk_l2norm, tfrag, knorm, tab, warm,    \
+                                              __VA_ARGS__)
+    const InvMore more{own, cap, keep};
+    if (use_own || cap.n) {
+      if (beta_dtype == GDN_BF16) GDN_INV_LAUNCH(uint16_t, true, more);
+      else GDN_INV_LAUNCH(float, true, more);
+    } else {
+      if (beta_dtype == GDN_BF16) GDN_INV_LAUNCH(uint16_t, false, NoArgs{});
+      else GDN_INV_LAUNCH(float, false, NoArgs{});
+    }
+#undef GDN_INV_LAUNCH
     int rc = check_launch("gdn_chunk_prefill(inverse)");
     if (rc) return rc;
   }
   auto launch = [&](int pass, int64_t blocks) {
-#define GDN_SEG_LAUNCH(BT)                                                                                           \
-  (pass == 1 ? seg_kernel<BT, uint16_t, 1>                                                                          \
-             : norm_mode == 1 ? seg_kernel<BT, uint16_t, 0, 1>                                                      \
-                              : norm_mode == 2 ? seg_kernel<BT, uint16_t, 0, 2> : seg_kernel<BT, uint16_t, 0>)      \
-      <<<(unsigned)blocks, sg::NT, 0, st>>>((const uint16_t*)q, q_stride, (const uint16_t*)k, k_stride,              \
-                                            (const uint16_t*)v, v_stride, g, (const BT*)beta, (uint16_t*)out, tab, Hqk, \
-                                            Hv, use_qk_l2norm, initial_state, state_rows, n_rows, final_state, trans,  \
-                                            tflags, tfrag, knorm, warm, gate)
+#define GDN_SEG(BT, PASS, NORM, FORM, ...)                                                                             \
+  seg_kernel<BT, uint16_t, PASS, NORM, FORM><<<(unsigned)blocks, sg::NT, 0, st>>>(                                     \
+      (const uint16_t*)q, q_stride, (const uint16_t*)k, k_stride, (const uint16_t*)v, v_stride, g, (const BT*)beta,    \
+      (uint16_t*)out, tab, __VA_ARGS__, Hqk, Hv, use_qk_l2norm, initial_state, state_rows, n_rows, final_state, trans, \
+      tflags, tfrag, knorm, warm, gate)
+#define GDN_SEG_OUT(BT, NORM)                                                                                          \
+  do {                                                                                                                 \
+    if (seg.walk) GDN_SEG(BT, 0, NORM, kOwnWalk, own);                                                                 \
+    else if (use_own) GDN_SEG(BT, 0, NORM, kOwnEven, own);                                                             \
+    else GDN_SEG(BT, 0, NORM, kFixed, NoArgs{});                                                                       \
+  } while (0)
+#define GDN_SEG_LAUNCH(BT)                                                                                             \
+  do {                                                                                                                 \
+    if (pass == 1) GDN_SEG(BT, 1, 0, kFixed, NoArgs{});                                                                 \
+    else if (norm_mode == 1) GDN_SEG_OUT(BT, 1);                                                                       \
+    else if (norm_mode == 2) GDN_SEG_OUT(BT, 2);                                                                       \
+    else GDN_SEG_OUT(BT, 0);                                                                                           \
+  } while (0)
     if (beta_dtype == GDN_BF16) GDN_SEG_LAUNCH(uint16_t);
     else GDN_SEG_LAUNCH(float);
 #undef GDN_SEG_LAUNCH
+#undef GDN_SEG_OUT
+#undef GDN_SEG
   };
   if (!seg.walk && lay.nslots > 0 && max_seq_chunks > lay.L) {  // segment summaries and their combination where no warm-up fits
     launch(1, lay.nslots * Hv * 2);
@@ -2514,20 +2563,20 @@ extern "C" int gdn_chunk_prefill_inverse(const void* k, int64_t k_stride, const 
     const int rc = check_launch("gdn_chunk_prefill_inverse(table)");
     if (rc) return rc;
   }
-  const SegTable tab{cu_seqlens, seq_chunk0, cu_seqlens ? seg0 : nullptr, nullptr, nseq, seq_len, (int)lay.L, 0, 0, nullptr, 1};
+  const SegTable tab{cu_seqlens, seq_chunk0, cu_seqlens ? seg0 : nullptr, nullptr, nseq, seq_len, (int)lay.L};
   uint8_t* tfrag = work + lay.off_tfrag;
   float* knorm = (float*)(work + lay.off_knorm);
   int* warm = (int*)(work + lay.off_warm);
   const int64_t items = total_chunks * Hv;
   const unsigned gi = (unsigned)((items + 3) / 4);
   if (beta_dtype == GDN_BF16)
-    inv_kernel<uint16_t><<<gi, pf::NT, 0, st>>>((const uint16_t*)k, k_stride, g, (const uint16_t*)beta, cu_seqlens,
-                                                seq_chunk0, nseq, seq_len, items, Hqk, Hv, use_qk_l2norm, tfrag,
-                                                knorm, tab, warm, CaptureArgs{}, KeepArgs{});
+    inv_kernel<uint16_t, false><<<gi, pf::NT, 0, st>>>((const uint16_t*)k, k_stride, g, (const uint16_t*)beta,
+                                                       cu_seqlens, seq_chunk0, nseq, seq_len, items, Hqk, Hv,
+                                                       use_qk_l2norm, tfrag, knorm, tab, warm, NoArgs{});
   else
-    inv_kernel<float><<<gi, pf::NT, 0, st>>>((const uint16_t*)k, k_stride, g, (const float*)beta, cu_seqlens,
-                                             seq_chunk0, nseq, seq_len, items, Hqk, Hv, use_qk_l2norm, tfrag, knorm,
-                                             tab, warm, CaptureArgs{}, KeepArgs{});
+    inv_kernel<float, false><<<gi, pf::NT, 0, st>>>((const uint16_t*)k, k_stride, g, (const float*)beta, cu_seqlens,
+                                                    seq_chunk0, nseq, seq_len, items, Hqk, Hv, use_qk_l2norm, tfrag,
+                                                    knorm, tab, warm, NoArgs{});
   int rc = check_launch("gdn_chunk_prefill_inverse(inverse)");
   if (rc) return rc;
   inv_records_expand_kernel<<<gi, 256, 0, st>>>(tfrag, knorm, items, t_out, use_qk_l2norm ? factor_out : nullptr);
