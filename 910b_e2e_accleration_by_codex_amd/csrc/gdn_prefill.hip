@@ -791,8 +791,9 @@ __device__ bool seq_warm_ok(const SegTable& tab, const int* __restrict__ warm, i
 // and the slowest head sets the output pass's time (T = 32768 with heads of every memory length: 64 + 28
 // steps where the mean is 70).  The output pass therefore takes the least number of steps T such that segments
 // of T chunks (a sequence's first) and T - w (the others) need at most kTargetItems workgroups over all
-// (sequence, key head) groups, w = the largest of the group's warm-ups at the fixed segments' ends; groups
-// with a head on the exact path keep their fixed segments.  (Per group, not per value head: the value
+// (sequence, key head) groups, w = the longest warm-up of the group's heads at any cut (longest_warm, left by the
+// summary pass in the flag of the head's first slot); groups with a head on the exact path, or with a warm-up
+// longer than a fixed segment, keep their fixed segments.  (Per group, not per value head: the value
 // heads of a key head then still run the same chunks side by side and share its q and K in L2.)  Every
 // workgroup works it out from the warm-up lengths by itself (about 1 us).
 constexpr int kMaxGroups = sg::kTargetItems;  // nseq Hqk <= nseq Hv <= kTargetItems
@@ -811,6 +812,8 @@ struct PlanItem {
 // A group with warm-ups of 3 or more chunks forgets less than e^-4 a chunk: its steps take W S in hi + lo and
 // cost 4/3 of the others (T = 8192: 5.2 against 4.0 us), so it runs 3/4 as many.
 __device__ __forceinline__ int plan_steps(int w, int steps) { return w >= 3 ? 3 * steps / 4 : steps; }
+// Warm-ups longer than this keep their group in the fixed segments.
+__device__ __forceinline__ int plan_cap(int L) { return L < 256 ? L : 256; }
 // Segments of a group of n chunks at `steps` steps, or a number past every target.
 __device__ __forceinline__ int plan_count(int n, int w, int steps, int L) {
   if (w == kExactGroup) return n <= L ? 1 : (n + L - 1) / L;
@@ -819,7 +822,8 @@ __device__ __forceinline__ int plan_count(int n, int w, int steps, int L) {
   const int d = steps - w;
   return d < 1 ? sg::kTargetItems + 1 : 1 + (n - steps + d - 1) / d;
 }
-__device__ PlanItem plan_segments(PlanSmem& P, const SegTable& tab, const int* __restrict__ warm, int Hqk, int Hv, int b) {
+__device__ PlanItem plan_segments(PlanSmem& P, const SegTable& tab, const int* __restrict__ warm,
+                                  const int* __restrict__ tflags, int Hqk, int Hv, int b) {
   const int t = threadIdx.x, r = Hv / Hqk, groups = tab.nseq * Hqk, entries = tab.first_slot(tab.nseq) * Hv;
   if (t < groups) {
     const int n = tab.nch(t / Hqk);
@@ -829,8 +833,13 @@ __device__ PlanItem plan_segments(PlanSmem& P, const SegTable& tab, const int* _
   if (t == 0) P.best = kExactGroup, P.cnt = 0;
   __syncthreads();
   for (int e = t; e < entries; e += sg::NT) {
-    const int wv = warm[e];
-    atomicMax(&P.w[tab.seq_of_slot(e / Hv) * Hqk + (e % Hv) / r], wv == 0 ? kExactGroup : wv);
+    const int ts = e / Hv, s = tab.seq_of_slot(ts);
+    int wv = warm[e] == 0 ? kExactGroup : 0;
+    if (wv == 0 && ts == tab.first_slot(s)) {  // (a head with an exact slot elsewhere has its own flag there)
+      wv = tflags[e];
+      if (wv > plan_cap(tab.L)) wv = kExactGroup;
+    }
+    atomicMax(&P.w[s * Hqk + (e % Hv) / r], wv);
   }
   __syncthreads();
   // candidates: from an even share up to what the fixed segments take
@@ -890,6 +899,36 @@ __device__ PlanItem plan_segments(PlanSmem& P, const SegTable& tab, const int* _
   }
   __syncthreads();  // the caller's chunk buffers take this memory
   return it;
+}
+// The longest warm-up (warm_before) that a cut anywhere in sequence s (head h) takes, or cap + 1 when one takes more
+// than cap chunks (whole workgroup; x: cap + sg::NT floats of LDS, best: one int of it).  The plan may cut anywhere:
+// with the warm-ups at the fixed segments' ends only, one beta above 1 in a chunk that none of those meets let a
+// segment cut after it warm up from the sequence's start (T = 32768 x 32 mixed heads: 430 us, up to 1299).
+__device__ int longest_warm(float* x, int* best, const SegTable& tab, const float* __restrict__ knorm, int Hv, int h,
+                            int s, int cap) {
+  const int t = threadIdx.x, n = tab.nch(s);
+  const int64_t first = tab.first_chunk(s);
+  int w = 0;
+  if (t == 0) *best = 0;
+  for (int c0 = 1; c0 < n; c0 += sg::NT) {  // thread t: the cut before chunk c0 + t; x[i]: chunk c0 - cap + i
+    __syncthreads();
+    for (int i = t; i < cap + sg::NT - 1; i += sg::NT) {
+      const int j = c0 - cap + i;
+      x[i] = j >= 0 && j < n ? knorm[((first + j) * Hv + h) * kr::FLOATS + kr::SUM] : 0.f;
+    }
+    __syncthreads();
+    const int c = c0 + t, most = c < cap ? c : cap;
+    if (c < n) {
+      float acc = 0.f;
+      int k = 0;
+      while (k < most && !(acc < sg::kWarmLog)) acc += x[cap + t - 1 - k++];
+      const int need = acc < sg::kWarmLog || c <= cap ? k : cap + 1;
+      w = need > w ? need : w;
+    }
+  }
+  atomicMax(best, w);
+  __syncthreads();
+  return *best;
 }
 // The least number of chunks before chunk c of sequence s (head h) whose summed log decay is below
 // kWarmLog, or c when there is none before the sequence's start (one wave; sums from the inverse
@@ -1513,8 +1552,9 @@ __device__ __forceinline__ void chain_part2(const SegBuf& B, ChainRegs& R, int l
 // (from the identity, without U), written into the slot; A is skipped when negligible.
 // Waves 0-3 (local) prepare chunk c+1's operands in one buffer (and store chunk c-1's outputs) while
 // waves 4-7 (chain) run chunk c from the other: two LDS barriers a chunk, met by both roles.
-// kForm (pass 0): kFixed, segments of L chunks; kOwnWalk, those of short sequences (every segment warms up as far back
-// as it takes); kOwnEven, those evened out by plan_segments (own.balance).  States kept aside (own.kept) need one of
+// kForm: kFixed, segments of L chunks; kOwnWalk, those of short sequences (every segment warms up as far back
+// as it takes); kOwnEven, those evened out by plan_segments (own.balance; in pass 1, the
+// warm-ups that the plan needs).  States kept aside (own.kept) need one of
 // the last two.  Each form runs a kernel without the others' code and arguments: with all of it in one kernel, 16
 // fresh prompts of 8 to 64 tokens x 32 heads through the layer took 49.0-49.3 us against 48.0-48.7 (over several
 // builds: where the code comes to lie moves these calls by up to 0.5 us), 353 tokens x 48 heads 26.2 against 25.9.
@@ -1540,7 +1580,7 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
   if (kPass == 0) {
     const int item = xcd_item(blockIdx.x, gridDim.x);
     if constexpr (kForm == kOwnEven) {
-      if (own.balance) plan = plan_segments(reinterpret_cast<PlanSmem&>(sm), tab, warm, Hqk, Hv, item);
+      if (own.balance) plan = plan_segments(reinterpret_cast<PlanSmem&>(sm), tab, warm, tflags, Hqk, Hv, item);
     }
     if (kForm == kOwnEven && plan.on) {
       if (plan.idle) return;
@@ -1566,7 +1606,14 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
     idx = ts - tab.first_slot(s);
     slot = ts;
     mode = (item & 1) ? kSegA : kSegB;
-    if (seq_warm_ok(tab, warm, Hv, h, s)) return;  // the output pass warms up instead
+    if (seq_warm_ok(tab, warm, Hv, h, s)) {  // the output pass warms up instead
+      if (kForm == kOwnEven && mode == kSegB && idx == 0) {
+        const int wl = longest_warm(reinterpret_cast<float*>(&sm), reinterpret_cast<int*>(sm.red), tab, knorm, Hv, h, s,
+                                    plan_cap(tab.L));
+        if (t == 0) tflags[(int64_t)slot * Hv + h] = wl;
+      }
+      return;
+    }
   }
   const int nch_s = tab.nch(s);
   const bool warm_path = kPass == 0 && slot >= 0 && seq_warm_ok(tab, warm, Hv, h, s);
@@ -2365,7 +2412,8 @@ int chunk_prefill_impl(const void* q, int64_t q_stride, const void* k, int64_t k
   const bool in_place = initial_state && initial_state == final_state && max_seq_chunks > seg.L;
   // segments evened out over the heads' warm-ups: where one round of workgroups holds them all and a segment is
   // long enough for the heads to differ by more than the planning costs
-  const int balance = !seg.walk && max_seq_chunks > lay.L && lay.L >= kBalanceMin && (int64_t)nseq * Hv <= sg::kTargetItems;
+  const int balance = !seg.walk && lay.nslots > 0 && max_seq_chunks > lay.L && lay.L >= kBalanceMin &&
+                      (int64_t)nseq * Hv <= sg::kTargetItems;
   const SegTable tab{cu_seqlens, seq_chunk0, cu_seqlens ? seg0 : nullptr, cu_seqlens ? order : nullptr, nseq, seq_len,
                      seg.L};
   const SegOwn own{balance, seg.walk, in_place ? (float*)(work + lay.off_kept) : nullptr, (int)lay.L};
@@ -2405,7 +2453,8 @@ int chunk_prefill_impl(const void* q, int64_t q_stride, const void* k, int64_t k
   } while (0)
 #define GDN_SEG_LAUNCH(BT)                                                                                             \
   do {                                                                                                                 \
-    if (pass == 1) GDN_SEG(BT, 1, 0, kFixed, NoArgs{});                                                                 \
+    if (pass == 1 && balance) GDN_SEG(BT, 1, 0, kOwnEven, own);                                                        \
+    else if (pass == 1) GDN_SEG(BT, 1, 0, kFixed, NoArgs{});                                                                 \
     else if (norm_mode == 1) GDN_SEG_OUT(BT, 1);                                                                       \
     else if (norm_mode == 2) GDN_SEG_OUT(BT, 2);                                                                       \
     else GDN_SEG_OUT(BT, 0);                                                                                           \

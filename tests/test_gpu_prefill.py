@@ -555,3 +555,39 @@ def test_chunk_prefill_balanced_segments(gdn, oracle, dev, lens, Hk, Hv, exact):
                 sl = slice(cu[i], cu[i + 1])
                 assert rel_l2(o[:, sl, h], o_ref[:, sl, h]) <= OUT_TOL, (i, h)
             assert rel_l2(s[i, h], s_ref[i, h]) <= STATE_TOL, (i, h)
+
+
+def test_chunk_prefill_balanced_segments_bound_their_warm_ups(gdn, dev):
+    """One beta above 1 anywhere in one fast head (no warm-up passes it) costs the call no more than a head on the
+    exact path does: a planned segment behind it that warmed up from the sequence's start would run hundreds of
+    steps, 3 times the whole call.  The states stay those of the call without it up to the chunk before (final states
+    of the other heads: the same bits or, where the plan differs, the path's rounding)."""
+    T, Hk, Hv = 32768, 16, 32
+    q, k, v, g, beta, _ = (x.to(dev) if x is not None else None for x in _gdn_inputs(T, Hk, Hv, seed=11, state=False))
+    g *= torch.logspace(-1.5, 1, Hv, device=dev)
+    h = Hv - 1  # the fastest
+
+    def run(beta):
+        return gdn.chunk_gated_delta_rule(q, k, v, g, beta, output_final_state=True, use_qk_l2norm_in_kernel=True)
+
+    def micros(beta):
+        best = float("inf")
+        for _ in range(4):
+            ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            ev[0].record()
+            run(beta)
+            ev[1].record()
+            ev[1].synchronize()
+            best = min(best, ev[0].elapsed_time(ev[1]))
+        return best
+
+    _, s_ref = run(beta)
+    base, worst = micros(beta), 0.0
+    for p in range(3, T // 64, 6):
+        b = beta.clone()
+        b[0, 64 * p + 7, h] = 1.5
+        worst = max(worst, micros(b))
+        if p % 60 == 3:
+            _, s = run(b)
+            assert rel_l2(s[0, :h], s_ref[0, :h]) <= STATE_TOL
+    assert worst < 2 * base, (worst, base)
