@@ -572,7 +572,7 @@ def test_chunk_prefill_balanced_segments_bound_their_warm_ups(gdn, dev):
 
     def micros(beta):
         best = float("inf")
-        for _ in range(4):
+        for _ in range(2):
             ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
             ev[0].record()
             run(beta)
@@ -583,11 +583,11 @@ def test_chunk_prefill_balanced_segments_bound_their_warm_ups(gdn, dev):
 
     _, s_ref = run(beta)
     base, worst = micros(beta), 0.0
-    for p in range(3, T // 64, 6):
+    for p in range(T // 64):  # a fast head's warm-up is one chunk: it meets p only from a cut right behind it
         b = beta.clone()
         b[0, 64 * p + 7, h] = 1.5
         worst = max(worst, micros(b))
-        if p % 60 == 3:
+        if p % 64 == 3:
             _, s = run(b)
             assert rel_l2(s[0, :h], s_ref[0, :h]) <= STATE_TOL
     assert worst < 2 * base, (worst, base)
