@@ -321,6 +321,7 @@ struct SegTable {
   }
 };
 
+constexpr int kMaxGroups = sg::kTargetItems;  // balanced calls: nseq Hqk <= nseq Hv <= kTargetItems
 // What only the calls with segments of other forms need (kForm, kMore below); the others' kernels do not take it.
 struct SegOwn {
   int balance;  // the output pass evens its segments out over the heads' warm-ups (plan_segments)
@@ -331,6 +332,10 @@ struct SegOwn {
   // sequence, since several segments are at least keep_len chunks).
   float* kept;
   int keep_len;
+  int share;   // balance: the calls' output steps over kTargetItems workgroups, in the plan's units
+  int* warms;  // balance: per (sequence of several segments, value head), as the plan takes them: its longest warm-up at
+               // any cut, and (kMaxGroups on) at the fixed segments' ends; kFixedGroup where the plan leaves them.  At
+               // 2 kMaxGroups, whether a head's fixed segments take so long that a plan may be worth its search
   __device__ __forceinline__ float* kept_state(const SegTable& tab, int s, int h, int Hv) const {
     return kept + ((int64_t)(tab.first_chunk(s) / keep_len) * Hv + h) * pf::D * pf::D;
   }
@@ -741,7 +746,10 @@ __global__ __launch_bounds__(pf::NT, 2) void inv_kernel(const uint16_t* __restri
   // the last chunk of a segment with a successor: that transition slot's warm-up length
   const int nch = tab.nch(cp.seq);
   bool walk = false;
-  if constexpr (kMore) walk = more.own.walk;
+  if constexpr (kMore) {
+    walk = more.own.walk;
+    if (more.own.balance && item == 0 && lane == 0) more.own.warms[2 * kMaxGroups] = 0;  // the summary pass sets it
+  }
   if (!walk && (cp.c + 1) % tab.L == 0 && cp.c + 1 < nch) {
     const int ts = tab.first_slot(cp.seq) + (cp.c + 1) / tab.L - 1;
     const int wv = use_l2 ? chunk_warm(g, beta, Hv, h, cp.t0, tab.L) : 0;
@@ -786,118 +794,212 @@ __device__ bool seq_warm_ok(const SegTable& tab, const int* __restrict__ warm, i
   }
   return true;
 }
+// The longest of the pair's warm-ups, 0 where a slot has none (one wave).
+__device__ int seq_warm_max(const SegTable& tab, const int* __restrict__ warm, int Hv, int h, int s) {
+  const int lane = threadIdx.x & 63;
+  const int ts0 = tab.first_slot(s), nslot = tab.first_slot(s + 1) - ts0;
+  float m = 0.f;
+  bool none = false;
+  for (int j = lane; j < nslot; j += 64) {
+    const int wv = warm[(int64_t)(ts0 + j) * Hv + h];
+    none |= wv == 0;
+    m = fmaxf(m, (float)wv);
+  }
+  return __builtin_amdgcn_ballot_w64(none) != 0 ? 0 : __builtin_amdgcn_readfirstlane((int)wave_max_fast(m));
+}
 
 // Balanced segments.  With L chunks a segment, a head whose warm-ups take w chunks runs L + w steps a segment,
 // and the slowest head sets the output pass's time (T = 32768 with heads of every memory length: 64 + 28
-// steps where the mean is 70).  The output pass therefore takes the least number of steps T such that segments
-// of T chunks (a sequence's first) and T - w (the others) need at most kTargetItems workgroups over all
-// (sequence, key head) groups, w = the longest warm-up of the group's heads at any cut (longest_warm, left by the
-// summary pass in the flag of the head's first slot); groups with a head on the exact path, or with a warm-up
-// longer than a fixed segment, keep their fixed segments.  (Per group, not per value head: the value
-// heads of a key head then still run the same chunks side by side and share its q and K in L2.)  Every
-// workgroup works it out from the warm-up lengths by itself (about 1 us).
-constexpr int kMaxGroups = sg::kTargetItems;  // nseq Hqk <= nseq Hv <= kTargetItems
+// steps where the mean is 70).  The output pass therefore takes the least time B such that segments of that time
+// need at most kTargetItems workgroups over all (sequence, key head) groups, w = the longest warm-up of the group's
+// heads at any cut (longest_warm, left by the summary pass); groups with a
+// head on the exact path, or with a warm-up longer than a fixed segment, keep their fixed segments.  (Per group, not
+// per value head: the value heads of a key head then still run the same chunks side by side and share its q and K
+// in L2.)  Times are in twelfths of an output step of a fast head; measured (constant decay, 16 to 48 heads, 10 and
+// 20 chunks a segment): bare rule 3.6 us, 4.9 for a head of warm-ups of 3 or more chunks (it forgets less than e^-4
+// a chunk and takes W S in hi + lo), 3.3 a warm-up step; with the fused norm, whose loads and stores the
+// warm-up steps don't have, 5.2, 6.5 and 3.1; one summary combined 4.2.  (With every step counted alike
+// the plan gave a fast head beside a slow one too much: T = 32768 x 48 through the layer 1053 -> 1087 us.)
+// The plan has to gain more than kPlanMargin (3 steps) over the fixed segments' slowest head: its search and the
+// warm-up lengths take 1 to 2 steps, and the counts above are off by as much.  Whole calls with mixed heads, fixed
+// segments -> plan: T = 32768 x 32 474 -> 422 us, 24001 x 16 236 -> 215, through the layer 32768 x 32 809 -> 741,
+// 16384 x 32 437 -> 400.  A call on which it is tried for nothing (all heads slow, on the exact path) loses 1%
+// (13000 x 32 384 -> 389).  Below kBalanceMin chunks a segment it lost more often than it won (mixed heads, 10 to 21
+// chunks: 6 of 16 calls 2 to 6% faster, 10 calls 1 to 5% slower), so it is not tried.  kPlanTry: a plan is searched only
+// where a head it may cut anew takes 4 steps longer than an even share of the output steps; the other calls
+// read that one word (8192 x 48 fast heads 144 -> 141.5 us).
 constexpr int kBalanceMin = 24;
+constexpr int kPlanMargin = 36, kPlanTry = 48;
 struct PlanSmem {
-  int w[kMaxGroups], n[kMaxGroups];  // the group's warm-up (kExactGroup: fixed segments) and its chunks
-  int best, s, hk, local, cnt;       // the step count found; this workgroup's group and place in it
+  int n[kMaxGroups];   // the group's chunks
+  int w[kMaxGroups];   // its longest warm-up at any cut (kFixedGroup: it keeps its fixed segments)
+  int wf[kMaxGroups];  // its longest warm-up at the fixed segments' ends (kFixedGroup: a head on the exact path)
+  int ok[8];
 };
-constexpr int kExactGroup = 1 << 30;
+constexpr int kFixedGroup = 1 << 30;
 struct PlanItem {
   bool on;        // false: the fixed segments stand
   bool idle;      // on, and no item is left for this workgroup
   int s, h;
-  int begin, end;  // chunks; end < 0: fixed segment number `begin` of a group on the exact path
+  int begin, end;  // chunks; end < 0: fixed segment number `begin` of a group that keeps them
 };
-// A group with warm-ups of 3 or more chunks forgets less than e^-4 a chunk: its steps take W S in hi + lo and
-// cost 4/3 of the others (T = 8192: 5.2 against 4.0 us), so it runs 3/4 as many.
-__device__ __forceinline__ int plan_steps(int w, int steps) { return w >= 3 ? 3 * steps / 4 : steps; }
+// a / d for 0 <= a < 2^21 and d >= 1: the reciprocal's and the product's roundings stay below the half added.
+__device__ __forceinline__ int small_div(int a, int d) {
+  return (int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)d));
+}
+template <bool kNorm>
+struct PlanCost {
+  static constexpr int FAST = 12, SLOW = kNorm ? 15 : 16, WARM = kNorm ? 7 : 11, COMBINE = kNorm ? 10 : 14;
+  static __device__ __forceinline__ int out(int w) { return w >= 3 ? SLOW : FAST; }
+  // chunks of the first segment and of the later ones of a group with warm-ups w, in time B
+  static __device__ __forceinline__ int first(int w, int B) { return w >= 3 ? B / SLOW : B / FAST; }
+  static __device__ __forceinline__ int later(int w, int B) { return first(w, B > w * WARM ? B - w * WARM : 0); }
+  static __device__ __forceinline__ int segs(int n, int L) { return n <= L ? 1 : small_div(n + L - 1, L); }
+  // the slowest of a group's m fixed segments (L chunks, n in all)
+  static __device__ __forceinline__ int fixed(int n, int m, int wf, int L) {
+    if (wf == kFixedGroup) return L * SLOW + m * COMBINE;
+    return (n < L ? n : L) * out(wf) + wf * WARM;
+  }
+  // segments of a group in time B, or a number past every target
+  static __device__ __forceinline__ int count(int n, int w, int B, int L) {
+    if (w == kFixedGroup) return segs(n, L);
+    const int n1 = first(w, B), d = later(w, B);
+    return n <= n1 ? 1 : d < 1 ? sg::kTargetItems + 1 : 1 + small_div(n - n1 + d - 1, d);
+  }
+};
 // Warm-ups longer than this keep their group in the fixed segments.
 __device__ __forceinline__ int plan_cap(int L) { return L < 256 ? L : 256; }
-// Segments of a group of n chunks at `steps` steps, or a number past every target.
-__device__ __forceinline__ int plan_count(int n, int w, int steps, int L) {
-  if (w == kExactGroup) return n <= L ? 1 : (n + L - 1) / L;
-  steps = plan_steps(w, steps);
-  if (n <= steps) return 1;
-  const int d = steps - w;
-  return d < 1 ? sg::kTargetItems + 1 : 1 + (n - steps + d - 1) / d;
-}
-__device__ PlanItem plan_segments(PlanSmem& P, const SegTable& tab, const int* __restrict__ warm,
-                                  const int* __restrict__ tflags, int Hqk, int Hv, int b) {
-  const int t = threadIdx.x, r = Hv / Hqk, groups = tab.nseq * Hqk, entries = tab.first_slot(tab.nseq) * Hv;
-  if (t < groups) {
-    const int n = tab.nch(t / Hqk);
-    P.n[t] = n;
-    P.w[t] = n <= tab.L ? kExactGroup : 0;  // (nothing known of its warm-ups: one fixed segment)
-  }
-  if (t == 0) P.best = kExactGroup, P.cnt = 0;
-  __syncthreads();
-  for (int e = t; e < entries; e += sg::NT) {
-    const int ts = e / Hv, s = tab.seq_of_slot(ts);
-    int wv = warm[e] == 0 ? kExactGroup : 0;
-    if (wv == 0 && ts == tab.first_slot(s)) {  // (a head with an exact slot elsewhere has its own flag there)
-      wv = tflags[e];
-      if (wv > plan_cap(tab.L)) wv = kExactGroup;
-    }
-    atomicMax(&P.w[s * Hqk + (e % Hv) / r], wv);
-  }
-  __syncthreads();
-  // candidates: from an even share up to what the fixed segments take
-  int64_t chunks = 0;
-  int wmax = 0, fixed = 0;
-  for (int i = 0; i < groups; ++i) {
-    const int n = P.n[i], w = P.w[i];
-    chunks += n;
-    if (w != kExactGroup) wmax = w > wmax ? w : wmax;
-    else fixed = n >= tab.L ? tab.L : n > fixed ? n : fixed;
-  }
-  int lo = (int)((chunks * r + sg::kTargetItems - 1) / sg::kTargetItems);
-  lo = lo > fixed ? lo : fixed;
-  // warm-ups of a sixteenth of a segment: nothing to even out
-  const int hi = 16 * wmax <= tab.L ? 0 : (tab.L + wmax) * 4 / 3;
-  if (__builtin_amdgcn_readfirstlane(hi) == 0) {
-    __syncthreads();
-    return PlanItem{false, false, 0, 0, 0, 0};
-  }
-  const int by = (hi - lo + sg::NT - 1) / sg::NT;
-  const int steps = lo + t * (by < 1 ? 1 : by);
-  if (steps > 0 && steps < hi) {
-    int sum = 0;
-    for (int i = 0; i < groups && sum <= sg::kTargetItems; ++i) sum += r * plan_count(P.n[i], P.w[i], steps, tab.L);
-    if (sum <= sg::kTargetItems) atomicMin(&P.best, steps);
-  }
-  __syncthreads();
+// Every workgroup works the plan out by itself, each wave over all groups (4 a lane); the waves try 8 values of B at
+// a time.
+template <bool kNorm>
+__device__ PlanItem plan_segments(PlanSmem& P, const SegTable& tab, const int* __restrict__ warms, int Hqk, int Hv, int b) {
+  using C = PlanCost<kNorm>;
+  const int t = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
+  const int r = Hv / Hqk, groups = tab.nseq * Hqk;
+  const int pairs = tab.nseq * Hv;
+  const bool many = tab.first_seg(tab.nseq) * Hv > sg::kTargetItems;  // fixed segments for more than one round
   PlanItem it{false, false, 0, 0, 0, 0};
-  const int T = __builtin_amdgcn_readfirstlane(P.best);
-  if (T != kExactGroup) {
-    it.on = true;
-    if (t < groups) {
-      int base = 0;
-      for (int i = 0; i < t; ++i) base += r * plan_count(P.n[i], P.w[i], T, tab.L);
-      const int c = r * plan_count(P.n[t], P.w[t], T, tab.L);
-      if (b >= base && b < base + c) {
-        P.s = t / Hqk;
-        P.hk = t % Hqk;
-        P.local = b - base;
-        P.cnt = c;
+  {  // calls with nothing to gain end here, before any barrier: each wave over all pairs, 4 a lane
+    const int4 pw = reinterpret_cast<const int4*>(warms)[lane], pf = reinterpret_cast<const int4*>(warms + kMaxGroups)[lane];
+    float fix = 0.f, lo = 0.f, load = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int i = 4 * lane + e;
+      if (i < pairs) {
+        const int n = tab.nch(small_div(i, Hv)), m = C::segs(n, tab.L);
+        const int wf = m == 1 ? 0 : e == 0 ? pf.x : e == 1 ? pf.y : e == 2 ? pf.z : pf.w;
+        const int w = m == 1 ? kFixedGroup : e == 0 ? pw.x : e == 1 ? pw.y : e == 2 ? pw.z : pw.w;
+        const float cost = (float)C::fixed(n, m, wf, tab.L);
+        fix = fmaxf(fix, cost);
+        if (w == kFixedGroup) lo = fmaxf(lo, cost);
+        load += (float)(n * C::out(wf) + (wf == kFixedGroup ? 0 : (m - 1) * wf * C::WARM));
       }
     }
-    __syncthreads();
-    it.idle = __builtin_amdgcn_readfirstlane(P.cnt) == 0;
-    if (!it.idle) {  // (wave-uniform values: scalar addresses and branches in the chunk loop)
-      it.s = __builtin_amdgcn_readfirstlane(P.s);
-      const int hk = __builtin_amdgcn_readfirstlane(P.hk), local = __builtin_amdgcn_readfirstlane(P.local);
-      const int n = __builtin_amdgcn_readfirstlane(P.n[it.s * Hqk + hk]), w = __builtin_amdgcn_readfirstlane(P.w[it.s * Hqk + hk]);
-      const int i = local / r;
-      it.h = hk * r + local % r;
-      const int Tg = plan_steps(w, T);
-      it.begin = i == 0 ? 0 : Tg + (i - 1) * (Tg - w);
-      it.end = i == 0 ? Tg : it.begin + Tg - w;
-      if (it.end > n) it.end = n;
-      if (w == kExactGroup) it.begin = i, it.end = -1;
-    }
+    fix = wave_max_fast(fix);
+    load = wave_sum_fast(load) / (float)sg::kTargetItems;
+    // (load: with the fixed segments' warm-ups, about what a plan's come to)
+    if (!many && __builtin_amdgcn_readfirstlane((int)(fix - fmaxf(wave_max_fast(lo), load))) < kPlanMargin) return it;
   }
-  __syncthreads();  // the caller's chunk buffers take this memory
+  int cn = 0, cw = kFixedGroup, cf = 0;  // thread t: (sequence, value head) t
+  if (t < pairs) {
+    cn = tab.nch(small_div(t, Hv));
+    const int pw = warms[t], pf = warms[kMaxGroups + t];
+    if (cn > tab.L) cw = pw, cf = pf;  // (else nothing is known of its warm-ups: one fixed segment)
+  }
+  if (t < kMaxGroups) P.w[t] = P.wf[t] = 0;
+  __syncthreads();
+  if (t < tab.nseq * Hv) {
+    const int g = small_div(t, r);  // = s Hqk + h / r
+    P.n[g] = cn;
+    atomicMax(&P.w[g], cw);
+    atomicMax(&P.wf[g], cf);
+  }
+  __syncthreads();
+  int n[4], w[4];
+  float chunks = 0.f, load = 0.f, fix = 0.f, lo_f = 0.f;  // (whole numbers below 2^24 where they matter)
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int i = 4 * lane + e;
+    const bool in = i < groups;
+    n[e] = in ? P.n[i] : 0;
+    w[e] = in ? P.w[i] : kFixedGroup;
+    const int wf = in ? P.wf[i] : 0, m = C::segs(n[e], tab.L);
+    const float cost = in ? (float)C::fixed(n[e], m, wf, tab.L) : 0.f;
+    chunks += (float)n[e];
+    load += (float)(n[e] * C::out(wf) + (m - 1) * (wf == kFixedGroup ? 0 : wf * C::WARM));
+    fix = fmaxf(fix, cost);
+    if (w[e] == kFixedGroup) lo_f = fmaxf(lo_f, cost);
+  }
+  __syncthreads();  // from here on only P.ok is used, and nothing after the search: the caller's buffers take this memory
+  lo_f = fmaxf(wave_max_fast(lo_f), ceilf(wave_sum_fast(chunks) * (float)(r * C::FAST) / (float)sg::kTargetItems));
+  int a = __builtin_amdgcn_readfirstlane((int)lo_f) - 1;  // B in (a, hi]
+  fix = wave_max_fast(fix);
+  // more than one round of fixed segments, dealt longest first: up to 3/2 of the mean load (batches of 4 and 8 prompts
+  // of 1000 to 9000 tokens, simulated: 1.06 to 1.36), and the plan always won there (8 of 3000 to 9000 x 16 mixed heads
+  // through the layer 662 -> 552 us, 667 -> 571)
+  if (many) fix = fmaxf(fix, 1.5f * (float)r * wave_sum_fast(load) / (float)sg::kTargetItems);
+  int hi = __builtin_amdgcn_readfirstlane((int)fix) - (many ? 0 : kPlanMargin);
+  bool found = false;
+  while (hi > a && (!found || hi - a > 4)) {  // the least B to a third of a step; hi - a shrinks every round
+    const int step = (hi - a + 7) / 8, B = a + step * (wv + 1) < hi ? a + step * (wv + 1) : hi;
+    float c = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c += 4 * lane + e < groups ? (float)C::count(n[e], w[e], B, tab.L) : 0.f;
+    c = wave_sum_fast(c);
+    if (lane == 0) P.ok[wv] = (float)r * c <= (float)sg::kTargetItems;
+    __syncthreads();
+    const uint64_t fits = __builtin_amdgcn_ballot_w64(lane < 8 && P.ok[lane & 7] != 0);
+    __syncthreads();
+    if (fits == 0) break;  // (the first round only: later ones end at a B that fits)
+    const int i = __builtin_ctzll(fits);
+    found = true;
+    if (a + step * (i + 1) < hi) hi = a + step * (i + 1);
+    a += step * i;
+  }
+  if (!found) return it;
+  it.on = true;
+  // this workgroup's group and its place in it
+  float cnt[4], mine = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    cnt[e] = 4 * lane + e < groups ? (float)(r * C::count(n[e], w[e], hi, tab.L)) : 0.f;
+    mine += cnt[e];
+  }
+  const float end = wave_incl_scan(mine);
+  const uint64_t past = __builtin_amdgcn_ballot_w64((float)b < end);
+  it.idle = past == 0;
+  if (!it.idle) {  // (wave-uniform values: scalar addresses and branches in the chunk loop)
+    const int src = __builtin_ctzll(past);
+    float local = (float)b - __shfl(end - mine, src, kWave);
+    int g = 4 * src, gn = 0, gw = 0;
+    bool done = false;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float c = __shfl(cnt[e], src, kWave);
+      const int ne = __shfl(n[e], src, kWave), we = __shfl(w[e], src, kWave);
+      if (!done) {
+        if (local < c) {
+          done = true;
+          g = 4 * src + e;
+          gn = ne;
+          gw = we;
+        } else {
+          local -= c;
+        }
+      }
+    }
+    g = __builtin_amdgcn_readfirstlane(g);
+    gn = __builtin_amdgcn_readfirstlane(gn);
+    gw = __builtin_amdgcn_readfirstlane(gw);
+    const int place = __builtin_amdgcn_readfirstlane((int)local), i = place / r;
+    it.s = g / Hqk;
+    it.h = g % Hqk * r + place % r;
+    const int n1 = C::first(gw, hi), d = C::later(gw, hi);
+    it.begin = i == 0 ? 0 : n1 + (i - 1) * d;
+    it.end = i == 0 ? n1 : it.begin + d;
+    if (it.end > gn) it.end = gn;
+    if (gw == kFixedGroup) it.begin = i, it.end = -1;
+  }
   return it;
 }
 // The longest warm-up (warm_before) that a cut anywhere in sequence s (head h) takes, or cap + 1 when one takes more
@@ -921,12 +1023,20 @@ __device__ int longest_warm(float* x, int* best, const SegTable& tab, const floa
     if (c < n) {
       float acc = 0.f;
       int k = 0;
-      while (k < most && !(acc < sg::kWarmLog)) acc += x[cap + t - 1 - k++];
+      for (int k0 = 0; k0 < most && !(acc < sg::kWarmLog); k0 += 4) {  // four loads at a time
+        float y[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) y[u] = k0 + u < most ? x[cap + t - 1 - k0 - u] : 0.f;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (k0 + u < most && !(acc < sg::kWarmLog)) acc += y[u], ++k;
+      }
       const int need = acc < sg::kWarmLog || c <= cap ? k : cap + 1;
       w = need > w ? need : w;
     }
   }
-  atomicMax(best, w);
+  w = (int)wave_max_fast((float)w);
+  if ((t & 63) == 0) atomicMax(best, w);
   __syncthreads();
   return *best;
 }
@@ -1578,9 +1688,10 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
   PlanItem plan{false, false, 0, 0, 0, 0};
   constexpr bool walk = kForm == kOwnWalk;
   if (kPass == 0) {
-    const int item = xcd_item(blockIdx.x, gridDim.x);
+    const int item = xcd_item(blockIdx.x, gridDim.x), jo = item / Hv;
+    int j = tab.order ? tab.order[jo] : jo;  // (jo within the order's part: nseg_max, or below the chunks' number)
     if constexpr (kForm == kOwnEven) {
-      if (own.balance) plan = plan_segments(reinterpret_cast<PlanSmem&>(sm), tab, warm, tflags, Hqk, Hv, item);
+      if (own.balance && own.warms[2 * kMaxGroups]) plan = plan_segments<kNorm != 0>(reinterpret_cast<PlanSmem&>(sm), tab, own.warms, Hqk, Hv, item);
     }
     if (kForm == kOwnEven && plan.on) {
       if (plan.idle) return;
@@ -1588,10 +1699,8 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
       h = plan.h;
       idx = plan.end < 0 ? plan.begin : 0;
     } else {
-      const int jo = item / Hv;
       h = item % Hv;
       if (jo >= tab.first_seg(tab.nseq)) return;
-      const int j = tab.order ? tab.order[jo] : jo;
       s = tab.seq_of_seg(j);
       idx = j - tab.first_seg(s);
     }
@@ -1606,14 +1715,26 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
     idx = ts - tab.first_slot(s);
     slot = ts;
     mode = (item & 1) ? kSegA : kSegB;
-    if (seq_warm_ok(tab, warm, Hv, h, s)) {  // the output pass warms up instead
-      if (kForm == kOwnEven && mode == kSegB && idx == 0) {
-        const int wl = longest_warm(reinterpret_cast<float*>(&sm), reinterpret_cast<int*>(sm.red), tab, knorm, Hv, h, s,
-                                    plan_cap(tab.L));
-        if (t == 0) tflags[(int64_t)slot * Hv + h] = wl;
+    bool warm_ok;
+    if constexpr (kForm == kOwnEven) {
+      const int wf = seq_warm_max(tab, warm, Hv, h, s);
+      warm_ok = wf != 0;
+      if (mode == kSegB && idx == 0) {
+        const int wl = !warm_ok ? 0 : longest_warm(reinterpret_cast<float*>(&sm), reinterpret_cast<int*>(sm.red), tab, knorm,
+                                                   Hv, h, s, plan_cap(tab.L));
+        if (t == 0) {
+          const bool free_cut = warm_ok && wl <= plan_cap(tab.L);
+          // (an exact head's fixed segments stand whatever the plan: only the others' can make one worth its search)
+          if (free_cut && PlanCost<false>::fixed(tab.nch(s), 2, wf, tab.L) - own.share >= kPlanTry)
+            own.warms[2 * kMaxGroups] = 1;
+          own.warms[s * Hv + h] = free_cut ? wl : kFixedGroup;
+          own.warms[kMaxGroups + s * Hv + h] = warm_ok ? wf : kFixedGroup;
+        }
       }
-      return;
+    } else {
+      warm_ok = seq_warm_ok(tab, warm, Hv, h, s);
     }
+    if (warm_ok) return;  // the output pass warms up instead
   }
   const int nch_s = tab.nch(s);
   const bool warm_path = kPass == 0 && slot >= 0 && seq_warm_ok(tab, warm, Hv, h, s);
@@ -2292,7 +2413,7 @@ int64_t seg_len(int64_t total_chunks, int nseq, int Hv) {
   return L < sg::kMinSeg ? sg::kMinSeg : L;
 }
 // Workspace layout: the segment table (nseq + 1 int32), the longest-first segment order (int32 per
-// segment, up to one per chunk), the transition flags (int32 per (slot,
+// segment, up to one per chunk), the plan's warm-ups (2 KiB, SegOwn::warms), the transition flags (int32 per (slot,
 // value head)), the warm-up lengths (int32 per (slot, value head)), the transition slots (128 KiB per
 // (slot, value head): A's bf16 hi + lo fragments, then B in fp32; layout in namespace tr), the copies of
 // initial states updated in place (64 KiB per (slot, value head), SegTable::kept), the
@@ -2300,7 +2421,7 @@ int64_t seg_len(int64_t total_chunks, int nseq, int Hv) {
 // its records of 64 K l2norm factors, the chunk's 64 g values and the lo flag (528 B per (chunk, value
 // head)), each part 256-byte aligned.
 struct SegLayout {
-  int64_t L, nslots, off_order, off_flags, off_warm, off_trans, off_kept, off_tfrag, off_knorm, bytes;
+  int64_t L, nslots, off_order, off_plan, off_flags, off_warm, off_trans, off_kept, off_tfrag, off_knorm, bytes;
 };
 SegLayout seg_layout(int64_t total_chunks, int nseq, int Hv) {
   auto up = [](int64_t x) { return (x + 255) / 256 * 256; };
@@ -2308,7 +2429,8 @@ SegLayout seg_layout(int64_t total_chunks, int nseq, int Hv) {
   l.L = seg_len(total_chunks, nseq, Hv);
   l.nslots = total_chunks / l.L;
   l.off_order = up(((int64_t)nseq + 1) * 4);
-  l.off_flags = l.off_order + up(((int64_t)nseq + total_chunks) * 4);  // segments: <= nseq + chunks
+  l.off_plan = l.off_order + up(((int64_t)nseq + total_chunks) * 4);  // segments: <= nseq + chunks
+  l.off_flags = l.off_plan + up((2 * kMaxGroups + 1) * 4);
   l.off_warm = l.off_flags + up(l.nslots * Hv * 4);
   l.off_trans = l.off_warm + up(l.nslots * Hv * 4);
   l.off_kept = l.off_trans + l.nslots * Hv * (int64_t)sg::kTrans * 4;
@@ -2413,10 +2535,12 @@ int chunk_prefill_impl(const void* q, int64_t q_stride, const void* k, int64_t k
   // segments evened out over the heads' warm-ups: where one round of workgroups holds them all and a segment is
   // long enough for the heads to differ by more than the planning costs
   const int balance = !seg.walk && lay.nslots > 0 && max_seq_chunks > lay.L && lay.L >= kBalanceMin &&
-                      (int64_t)nseq * Hv <= sg::kTargetItems;
+                      (int64_t)nseq * Hv <= sg::kTargetItems && total_chunks < (1 << 20);
   const SegTable tab{cu_seqlens, seq_chunk0, cu_seqlens ? seg0 : nullptr, cu_seqlens ? order : nullptr, nseq, seq_len,
                      seg.L};
-  const SegOwn own{balance, seg.walk, in_place ? (float*)(work + lay.off_kept) : nullptr, (int)lay.L};
+  const SegOwn own{balance, seg.walk, in_place ? (float*)(work + lay.off_kept) : nullptr, (int)lay.L,
+                   balance ? (int)((total_chunks * Hv * PlanCost<false>::FAST + sg::kTargetItems - 1) / sg::kTargetItems) : 0,
+                   (int*)(work + lay.off_plan)};
   const bool use_own = seg.walk || balance || in_place;
   KeepArgs keep{};
   if (in_place) keep = KeepArgs{(nseq * Hv + 7) / 8 * 8, initial_state, state_rows, n_rows};
