@@ -176,9 +176,9 @@ int gdn_chunk_prefill_generic_ws(const void* q, int64_t q_stride, const void* k,
 /*
  * Bytes of device workspace gdn_chunk_prefill needs for `total_chunks` 64-token chunks of `nseq`
  * sequences and Hv value heads (-1 for bad sizes): the segment table and flags (a few bytes per
- * sequence and per segment), the fp32 transition maps of the segments that have a successor (at
- * most 32 MiB: sequences are cut into segments so that at most about 256 (segment, value head)
- * items exist) and the intra-chunk inverse's output (10.5 KiB per (chunk, value head): T diag(beta) as
+ * sequence and per segment), the transition maps of the segments that have a successor and copies of
+ * initial states that are updated in place (at most 32 + 16 MiB: sequences are cut into segments so that at
+ * most about 256 (segment, value head) items exist) and the intra-chunk inverse's output (10.5 KiB per (chunk, value head): T diag(beta) as
  * bf16 hi + lo, the K row factors, g and a flag).
  */
 int64_t gdn_chunk_prefill_workspace_bytes(int64_t total_chunks, int nseq, int Hv);
@@ -297,18 +297,18 @@ int gdn_chunk_prefill_rows_gated(const void* q, int64_t q_stride, const void* k,
 
 /*
  * gdn_chunk_prefill_rows without a workspace argument and without any allocation: the kernels'
- * workspace is a static device array of GDN_NOALLOC_SCRATCH_BYTES (256 MiB) that the library holds on
+ * workspace is a static device array of GDN_NOALLOC_SCRATCH_BYTES (273 MiB) that the library holds on
  * every GPU it runs on until the process ends.  A call whose
  * gdn_chunk_prefill_workspace_bytes(total_chunks, nseq, Hv) exceeds it is rejected with GDN_EINVAL
- * before any launch (the workspace is at most about 32 MiB plus 10.5 KiB per (chunk, value head): 256 MiB
- * holds e.g. 44,416 tokens at Hv = 32).  Every
+ * before any launch (the workspace is at most about 48 MiB plus 10.5 KiB per (chunk, value head): one
+ * sequence of 44,928 tokens at Hv = 32 fits, 30,656 at 48, 88,768 at 16).  Every
  * call on one GPU shares that GPU's array: calls that overlap on one GPU (other streams, other host
  * threads) race and give wrong results -- order them on one stream.  The array needs no clearing
  * (every record a call uses, the same call writes first).
  * No counterpart in the reference: for callers that cannot allocate (code under HIP graph capture,
  * serving loops, harnesses that forbid hipMalloc).
  */
-#define GDN_NOALLOC_SCRATCH_BYTES (256ll << 20)
+#define GDN_NOALLOC_SCRATCH_BYTES (273ll << 20)
 int gdn_chunk_prefill_noalloc(const void* q, int64_t q_stride, const void* k, int64_t k_stride,
                               const void* v, int64_t v_stride, const float* g, const void* beta,
                               int beta_dtype, const float* initial_state, float* final_state,

@@ -149,3 +149,30 @@ def test_prefill_layer_entry_host_checks(lib):
     # not match its length -- refused on the host, no launch (a launch would fail here: no GPU)
     assert call(chunk0=None) == 1 and b"seq_chunk0" in h.gdn_last_error()
     assert call(cu=None, chunk0=None, seq_len=T // nseq) == 1 and b"total_chunks" in h.gdn_last_error()
+
+
+def test_noalloc_scratch_holds_what_fitted_before_states_were_kept_aside(lib):
+    """The workspace grew by the copies of initial states updated in place, a longer segment order and the plan's
+    warm-ups; the static scratch of gdn_chunk_prefill_noalloc grew with it: every call whose workspace without those
+    (the formula below) was within 256 MiB still fits."""
+    h = lib.lib()
+    text = open(HEADER).read()
+    m = re.search(r"GDN_NOALLOC_SCRATCH_BYTES \((\d+)ll << 20\)", text)
+    scratch = int(m.group(1)) << 20
+
+    def up(x):
+        return (x + 255) // 256 * 256
+
+    def without(total, nseq, Hv):
+        pairs = nseq * Hv
+        work = nseq * (256 // pairs) if pairs <= 256 else None
+        L = max(2, -(-total // work) if work else -(-total * Hv // 256))
+        slots = total // L
+        return (up((nseq + 1) * 4) + up((nseq + total // L) * 4) + 2 * up(slots * Hv * 4) + slots * Hv * (128 << 10)
+                + total * Hv * (10 * 1024 + 528))
+
+    for Hv in (1, 4, 16, 32, 48, 64, 128, 300):
+        for nseq in (1, 2, 5, 16, 200):
+            for total in sorted({n for f in (1, 3) for n in range(nseq, 30000, 37 * f)} | set(range(300, 1500))):
+                if without(total, nseq, Hv) <= 256 << 20:
+                    assert h.gdn_chunk_prefill_workspace_bytes(total, nseq, Hv) <= scratch, (total, nseq, Hv)

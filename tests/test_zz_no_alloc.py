@@ -103,3 +103,28 @@ def test_noalloc_prefill_under_graph_capture(gdn, dev):
         torch.cuda.synchronize()
         assert torch.equal(out, o_ref) and torch.equal(fin, f_ref), f"replay {i}"
         assert torch.equal(o_e, o_ref) and torch.equal(f_e, f_ref), f"eager call {i}"
+
+
+@pytest.mark.gpu
+def test_noalloc_prefill_at_its_longest(gdn, dev):
+    """44,352 tokens of 32 value heads (what 256 MiB held before states updated in place were kept aside), states in
+    place: bit-identical to the workspace entry point."""
+    L = importlib.import_module(PKG_NAME + "._lib")
+    T, Hk, Hv, D = 44352, 16, 32, 128
+    r = torch.Generator(device=dev).manual_seed(7)
+    q, k, v = (torch.randn(T, H, D, generator=r, device=dev).to(torch.bfloat16) for H in (Hk, Hk, Hv))
+    beta = torch.sigmoid(torch.randn(T, Hv, generator=r, device=dev)).to(torch.bfloat16)
+    g = -torch.rand(T, Hv, generator=r, device=dev) * torch.logspace(-2, 0, Hv, device=dev)
+    s0 = 0.02 * torch.randn(1, Hv, D, D, generator=r, device=dev)
+    work = torch.empty(int(L.lib().gdn_chunk_prefill_workspace_bytes(T // CHUNK, 1, Hv)), dtype=torch.uint8, device=dev)
+    got = []
+    for name in ("gdn_chunk_prefill_rows", "gdn_chunk_prefill_noalloc"):
+        out, state = torch.empty(T, Hv, D, dtype=torch.bfloat16, device=dev), s0.clone()
+        args = [L.ptr(q), q.stride(0), L.ptr(k), k.stride(0), L.ptr(v), v.stride(0), L.ptr(g), L.ptr(beta), L.BF16,
+                L.ptr(state), L.ptr(state), None, 1, L.ptr(out), T, None, None, T // CHUNK, 1, T, Hk, Hv, D, L.BF16, 1]
+        if name.endswith("rows"):
+            args += [L.ptr(work), work.numel()]
+        L.call(name, *args, L.stream_of(q))
+        got.append((out, state))
+    torch.cuda.synchronize()
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
