@@ -6,7 +6,8 @@
 // HBM-bound on the cache (read once).  Launches:
 //   1. attn_prep_kernel, only when the projection comes as split-K partials: one wave per (slot, head
 //      row).  RMSNorm (fp32, (1 + w), bf16) of the q and k rows, rotary on the first rd dims (fp32,
-//      bf16), q kept in fp32 for the scores, k and v written into the cache at the slot's position.
+//      bf16), q handed on in fp32 (bf16 values: the scores take them as such), k and v written into the cache at
+//      the slot's position.
 //      With a bf16 projection the split kernel's workgroups do that themselves (each its kv head's q
 //      rows, the one holding the slot's position also k and v), under the latency of their cache loads.
 //   2. attn_split_kernel: one workgroup per (256-token split, kv head, slot) with the kv head's G query
@@ -352,16 +353,18 @@ __global__ __launch_bounds__(attn::split_threads(HD), 4) void attn_split_kernel(
 #pragma unroll
     for (int i = 0; i < 4; ++i) D[i] = mma(a[i], q, D[i]);
   }
-  // ---- V (tokens past the range: the last row, whose probability is 0), into the registers K leaves
+  // ---- V, into the registers K leaves.  Rows past the range read as zero (a buffer of the split's rows in range: loads
+  // past it return 0): their probability is 0, and 0 times an infinity of a row taken in their place would be NaN
   u32v vr[2][8];
   {
-    const uint16_t* vp = vc + (((int64_t)n * kv + j) * T + t0) * HD + d0 + EV * c;
+    const auto rows = __builtin_amdgcn_make_buffer_rsrc(vc + (((int64_t)n * kv + j) * T + t0) * HD, 0, cnt * HD * 2, 0x00027000);
+    const int at = ((64 * th + 16 * g4) * HD + d0 + EV * c) * 2;
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int tk = 64 * th + 16 * g4 + 8 * u + e, tc = tk < cnt ? tk : cnt - 1;
-        vr[u][e] = __builtin_nontemporal_load(reinterpret_cast<const u32v*>(vp + (int64_t)tc * HD));
+      for (int e = 0; e < 8; ++e) {  // non-temporal
+        if constexpr (EV == 8) vr[u][e] = __builtin_amdgcn_raw_buffer_load_b128(rows, at + (8 * u + e) * HD * 2, 0, 2);
+        else vr[u][e] = __builtin_amdgcn_raw_buffer_load_b64(rows, at + (8 * u + e) * HD * 2, 0, 2);
       }
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -405,10 +408,8 @@ __global__ __launch_bounds__(attn::split_threads(HD), 4) void attn_split_kernel(
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int tk = 64 * th + 16 * g4 + 8 * u + e;
-        if ((tk < cnt ? tk : cnt - 1) - 64 * th == prel) vr[u][e] = *reinterpret_cast<const u32v*>(&vnew[d0 + EV * c]);
-      }
+      for (int e = 0; e < 8; ++e)
+        if (16 * g4 + 8 * u + e == prel) vr[u][e] = *reinterpret_cast<const u32v*>(&vnew[d0 + EV * c]);
   }
   f32x4 O[EV];
 #pragma unroll

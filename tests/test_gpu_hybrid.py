@@ -201,6 +201,32 @@ def test_gqa_decode_attention_wave_and_split_edges(gdn, dev, nh, kv, hd, T):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("nh,kv,hd", [(6, 1, 256), (8, 2, 128), (4, 4, 64)])
+def test_gqa_decode_attention_infinite_values(gdn, dev, nh, kv, hd):
+    """An infinity in the new token's value row (the last one in range) stays one in the output's column, at counts
+    that do and do not fill a wave's 64 tokens; the other columns match the fp32 loop."""
+    from importlib import import_module
+    cb = import_module(PKG_NAME + ".cb_engine")
+    pos, T = [0, 5, 62, 63, 64, 126, 255, 300], 516
+    N, rd, eps = len(pos), hd // 4, 1e-6
+    g_ = torch.Generator().manual_seed(hd)
+    bf = torch.bfloat16
+    proj = torch.randn(N, (2 * nh + 2 * kv) * hd, generator=g_).to(bf)
+    proj[:, (2 * nh + kv) * hd + 3] = float("inf")  # column 3 of the first kv head
+    qn, kn = (0.1 * torch.randn(hd, generator=g_)).to(bf), (0.1 * torch.randn(hd, generator=g_)).to(bf)
+    inv = 1.0 / (10000.0 ** (torch.arange(0, rd, 2).float() / rd))
+    kt, vc = torch.randn(N, kv, hd, T, generator=g_).to(bf), torch.randn(N, kv, T, hd, generator=g_).to(bf)
+    ref = _attn_reference(proj, torch.tensor(pos), qn, kn, inv, kt, vc, nh, kv, hd, rd, eps).view(N, nh, hd)
+    out = cb.gqa_decode_attention(proj.to(dev), torch.tensor(pos, device=dev), qn.to(dev), kn.to(dev), inv.to(dev),
+                                  kt.to(dev), vc.to(dev), nh, kv, hd, rd, eps).cpu().float().view(N, nh, hd)
+    first = torch.zeros(nh, hd, dtype=torch.bool)
+    first[:nh // kv, 3] = True
+    assert bool((out[:, first] == float("inf")).all())
+    for n in range(N):  # bf16 probabilities and output: 2^-9 a value
+        assert rel_l2(out[n][~first], ref[n][~first]) <= OUT_TOL, pos[n]
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("nh,kv,hd,H", [(4, 2, 64, 512), (24, 4, 256, 5120)])
 def test_gqa_decode_attention_from_partials(gdn, dev, nh, kv, hd, H):
     """The attention fed the q|gate|k|v projection's split-K partials gives exactly what it gives on the
