@@ -256,6 +256,10 @@ constexpr float kNegligibleLog = -44.3614f;  // ln(2^-64): a segment map A_j thi
 // part is lost in the rounding the chain makes anyway (unless the state shrank by more than 2^7 over
 // the warm-up: new tokens contributing under 1/128 of the state they replace).
 constexpr float kWarmLog = -11.0904f;        // ln(2^-16)
+// Where the exact path would take the head (its warm-up is longer than the segments the host cuts) and a short sequence
+// walks instead, the dropped map is bounded by fp32's own rounding: with kWarmLog, an initial state 10^4 times the
+// final one was lost from heads that forget e^-3 a chunk (353 tokens: 1.6e-3 of the final state).
+constexpr float kDeepLog = -16.6355f;        // ln(2^-24)
 // A chunk whose decay over its tokens is slight (e^{G_last} above e^-4) passes much of the state it
 // receives on: the bf16 rounding of the W S operands then accumulates over the chunks (to 1e-3 of
 // the state over 8192 tokens of decay ~0.002 a token), or, from a large initial state that decays
@@ -331,7 +335,7 @@ struct SegOwn {
   // that no launch order bounds; a sequence's copy is [Hv, D, D] fp32 at first_chunk / keep_len (one per
   // sequence, since several segments are at least keep_len chunks).
   float* kept;
-  int keep_len;
+  int keep_len;  // the length of a segment where the call takes summaries (chunks)
   int share;   // balance: the calls' output steps over kTargetItems workgroups, in the plan's units
   int* warms;  // balance: per (sequence of several segments, value head), as the plan takes them: its longest warm-up at
                // any cut, and (kMaxGroups on) at the fixed segments' ends; kFixedGroup where the plan leaves them.  At
@@ -1041,9 +1045,9 @@ __device__ int longest_warm(float* x, int* best, const SegTable& tab, const floa
   return *best;
 }
 // The least number of chunks before chunk c of sequence s (head h) whose summed log decay is below
-// kWarmLog, or c when there is none before the sequence's start (one wave; sums from the inverse
+// `bound`, or c when there is none before the sequence's start (one wave; sums from the inverse
 // kernel's records, 64 chunks at a time).
-__device__ int warm_before(const SegTable& tab, const float* __restrict__ knorm, int Hv, int h, int s, int c) {
+__device__ int warm_before(const SegTable& tab, const float* __restrict__ knorm, int Hv, int h, int s, int c, float bound) {
   const int lane = threadIdx.x & 63;
   const int64_t first = tab.first_chunk(s);
   float acc = 0.f;
@@ -1051,7 +1055,7 @@ __device__ int warm_before(const SegTable& tab, const float* __restrict__ knorm,
     const int back = c0 + lane;  // chunk c - 1 - back
     const float x = back < c ? knorm[((first + c - 1 - back) * Hv + h) * kr::FLOATS + kr::SUM] : 0.f;
     const float sum = acc + wave_incl_scan(x);
-    const uint64_t hit = __builtin_amdgcn_ballot_w64(back < c && sum < sg::kWarmLog);
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(back < c && sum < bound);
     if (hit) return c0 + __builtin_ctzll(hit) + 1;
     acc = __shfl(sum, 63, kWave);
   }
@@ -1777,8 +1781,12 @@ __global__ __launch_bounds__(sg::NT, 1) void seg_kernel(
   }
   constexpr bool need_q = kPass == 0;
   // pass 0 after a warm-up: the chain starts from zero w0 chunks before the segment, without outputs
-  const int w0 = even ? (c_begin > 0 ? warm_before(tab, knorm, Hv, h, s, c_begin) : 0)
-                      : (kPass == 0 && warm_path) ? warm[(int64_t)slot * Hv + h] : 0;
+  int w0 = (kPass == 0 && warm_path) ? warm[(int64_t)slot * Hv + h] : 0;
+  if (even && c_begin > 0) {
+    w0 = warm_before(tab, knorm, Hv, h, s, c_begin, sg::kWarmLog);
+    if constexpr (kForm == kOwnWalk)
+      if (w0 > own.keep_len && w0 < c_begin) w0 = warm_before(tab, knorm, Hv, h, s, c_begin, sg::kDeepLog);
+  }
   const int cb0 = c_begin - w0, ntot = n + w0;
   const int chunk_slot0 = tab.first_chunk(s) + cb0;
   auto tfr = [&](int c) { return tfrag + ((int64_t)(chunk_slot0 + c) * Hv + h) * tf::BYTES; };
