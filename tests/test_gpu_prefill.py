@@ -499,15 +499,34 @@ def test_chunk_prefill_short_sequences_walk(gdn, oracle, dev, lens, n_rows, Hk, 
         assert torch.equal(sd[spare].cpu(), slots[spare])
 
 
-@pytest.mark.parametrize("lens,Hk,Hv,scale", [([353] * 9, 16, 48, 0.01), ([353, 100, 700] * 3, 16, 48, 1.0),
-                                              ([2000, 0, 1500, 64] * 3, 16, 32, 0.01), ([16447], 16, 32, 0.3)])
-def test_chunk_prefill_states_in_place_match_separate_buffers(gdn, dev, lens, Hk, Hv, scale):
-    """More segments than the chip runs at once, states updated in their slot rows: every segment that starts from
-    its sequence's initial state finds it whole, also when the last segment has already written the row.  The same
-    bits as with separate initial and final buffers, the rows of empty sequences and spare rows included."""
+def _segments(lens, Hv):
+    """How the library cuts a packed batch: (chunks a segment, (segment, value head) items).  256 items fill the chip."""
+    chunks, pairs = [-(-n // 64) for n in lens], len(lens) * Hv
+    total = sum(chunks)
+    L = max(2, -(-total // (len(lens) * (256 // pairs))) if pairs <= 256 else -(-total * Hv // 256))
+    return L, sum(max(1, -(-n // L)) for n in chunks) * Hv
+
+
+@pytest.mark.parametrize("lens,Hk,Hv,scale,rounds", [
+    ([3000] + [64] * 12, 16, 32, 0.01, 2),            # slow decay: the summaries and their combination
+    ([2000, 0, 1500, 64] * 3, 16, 32, 0.01, 2),
+    ([3000] + [64] * 12, 16, 32, 1.0, 2),             # fast decay: warm-ups
+    ([1200] + [300] * 8, 16, 32, 0.3, 2),             # short sequences that walk, every memory length
+    ([9000, 4000, 4000, 4000], 16, 32, 0.3, 2),       # evened out over the warm-ups
+    ([300, 130, 130], 8, 16, 0.01, 1),                # one-chunk segments: the copies lie closest together
+    ([16447], 16, 32, 0.3, 1),
+    ([353] * 9, 16, 48, 0.01, 0), ([353, 100, 700] * 3, 16, 48, 1.0, 0),  # one segment each: nothing is kept aside
+])
+def test_chunk_prefill_states_in_place_match_separate_buffers(gdn, dev, lens, Hk, Hv, scale, rounds):
+    """Sequences of several segments (rounds 2: more segments than the chip runs at once), states updated in their
+    slot rows: every segment that starts from its sequence's initial state finds it whole, also when the last segment
+    has already written the row.  The same bits as with separate initial and final buffers, the rows of empty sequences
+    and spare rows included."""
+    L, items = _segments(lens, Hv)
+    assert (-(-max(lens) // 64) > L) == (rounds > 0) and (items > 256) == (rounds != 1)
     T = sum(lens)
     q, k, v, g, beta, _ = (x.to(dev) if x is not None else None for x in _gdn_inputs(T, Hk, Hv, seed=T, state=False))
-    g *= scale
+    g *= scale * (torch.logspace(-1.3, 1, Hv, device=dev) if scale == 0.3 else 1.0)
     cu = [0]
     for n in lens:
         cu.append(cu[-1] + n)
@@ -526,16 +545,24 @@ def test_chunk_prefill_states_in_place_match_separate_buffers(gdn, dev, lens, Hk
     assert torch.equal(inplace, separate)
 
 
-@pytest.mark.parametrize("lens,Hk,Hv,exact", [([16447], 16, 32, False), ([20000, 9000, 0, 3000], 8, 16, True),
-                                              ([16384], 8, 16, True)])
-def test_chunk_prefill_balanced_segments(gdn, oracle, dev, lens, Hk, Hv, exact):
+@pytest.mark.parametrize("lens,Hk,Hv,exact,uniform", [
+    ([16447], 16, 32, False, False), ([20000, 9000, 0, 3000], 8, 16, True, False), ([24640], 8, 16, True, False),
+    ([16384], 8, 16, True, False),  # 16 chunks a segment: too short for the plan, fixed segments
+    ([24640], 8, 16, False, True), ([24640], 16, 16, True, True), ([12320] * 2, 8, 16, True, True),
+    ([9000, 4000, 4000, 4000], 16, 32, False, False),  # more fixed segments than one round holds
+])
+def test_chunk_prefill_balanced_segments(gdn, oracle, dev, lens, Hk, Hv, exact, uniform):
     """Heads of very different memory lengths in segments long enough to be evened out over their warm-ups
-    (1 to about 20 chunks): some groups run more, shorter segments than others; with `exact`, one head has no
-    warm-up at all and another a beta above 1 (a segment near it starts from the sequence's start), beside heads of
-    the same key head that warm up.  Initial states; every (sequence, head) against the oracle."""
+    (1 to about 20 chunks): some groups run more, shorter segments than others, in packed and uniform batches.  One
+    fast head decays nothing over a stretch between two fixed segments' ends; with `exact`, one head has no warm-up at
+    all and another a beta above 1, beside heads of the same key head that warm up.  Initial states; every (sequence,
+    head) against the oracle."""
+    L, _ = _segments(lens, Hv)
+    assert (L >= 24) == (lens != [16384]) and -(-max(lens) // 64) > L  # the plan is tried from 24 chunks a segment
     T = sum(lens)
     q, k, v, g, beta, _ = _gdn_inputs(T, Hk, Hv, seed=T + Hv, state=False)
     g *= torch.logspace(-1.3, 1, Hv)
+    g[0, 64 * (L + 3):64 * (L + 3 + L // 2), Hv - 2] = 0.0
     if exact:
         g[..., 3] *= 0.001
         beta[0, 5000, Hv - 1] = 1.5
@@ -546,9 +573,12 @@ def test_chunk_prefill_balanced_segments(gdn, oracle, dev, lens, Hk, Hv, exact):
     r = Hv // Hk
     o_ref, s_ref = oracle.chunk_gated_delta_rule_varlen(_rep(q, r), _rep(k, r), v, g, beta, torch.tensor(cu), 64, s0,
                                                         True, True)
-    o, s = gdn.chunk_gated_delta_rule(q.to(dev), k.to(dev), v.to(dev), g.to(dev), beta.to(dev), initial_state=s0.to(dev),
-                                      output_final_state=True, cu_seqlens=cu, use_qk_l2norm_in_kernel=True)
-    o, s = o.cpu(), s.cpu()
+    args = [x.to(dev) for x in (q, k, v, g, beta)]
+    if uniform:
+        args = [x.view(len(lens), lens[0], *x.shape[2:]) for x in args]
+    o, s = gdn.chunk_gated_delta_rule(*args, initial_state=s0.to(dev), output_final_state=True,
+                                      cu_seqlens=None if uniform else cu, use_qk_l2norm_in_kernel=True)
+    o, s = o.cpu().view(1, T, Hv, 128), s.cpu()
     for i in range(len(lens)):
         for h in range(Hv):
             if lens[i]:
