@@ -207,9 +207,9 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(attn::Src proj, const in
 //
 // What bounds it: HBM, and how K's rows meet the cache lines (a row of T bf16 values is a whole number of
 // lines only where T % 64 == 0).  16 slots of 24 / 4 heads of 256, whole calls (152 MB):
-//   contexts 512..4096, T = 4112: 54.5 us with prep and combine kernels around a v_dot2 split kernel of
-//     55 KB of LDS whose V loads waited for the softmax, 43 us here; T = 4160: 49 -> 35 us;
-//   contexts 1024: 30.8 -> 24 us; 4096: 71 -> 60 us; 8176: 113 -> 102 us (5.3 TB/s).
+//   contexts 512..4096, T = 4112: 51.6 us with prep and combine kernels around a v_dot2 split kernel of 55 KB of LDS
+//   whose V loads waited for the softmax, 38.0 us here; T = 4160: 49.9 -> 36.4 us;
+//   contexts 1024: 29.1 -> 23.5 us; 4096: 69.1 -> 54.5 us; 8176: 111.4 -> 88 us (6.1 TB/s).
 // On the way: every K and V load up front on v_dot2 (28 VALU instructions per 16 bytes loaded at G = 6, 2 waves a
 // SIMD) 68 us; the same on MFMA 59 us; 128-token splits, whose K pieces are half as long, 47 us.
 //
