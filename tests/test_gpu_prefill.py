@@ -603,8 +603,8 @@ def test_chunk_prefill_short_sequences_keep_a_large_initial_state(gdn, oracle, d
 def test_chunk_prefill_balanced_segments_bound_their_warm_ups(gdn, dev):
     """One beta above 1 anywhere in one fast head (no warm-up passes it) costs the call no more than a head on the
     exact path does: a planned segment behind it that warmed up from the sequence's start would run hundreds of
-    steps, 3 times the whole call.  The states stay those of the call without it up to the chunk before (final states
-    of the other heads: the same bits or, where the plan differs, the path's rounding)."""
+    steps, 3 times the whole call.  The other heads' final states stay where they were, to the path's rounding (the plan
+    may differ)."""
     T, Hk, Hv = 32768, 16, 32
     q, k, v, g, beta, _ = (x.to(dev) if x is not None else None for x in _gdn_inputs(T, Hk, Hv, seed=11, state=False))
     g *= torch.logspace(-1.5, 1, Hv, device=dev)
@@ -613,9 +613,9 @@ def test_chunk_prefill_balanced_segments_bound_their_warm_ups(gdn, dev):
     def run(beta):
         return gdn.chunk_gated_delta_rule(q, k, v, g, beta, output_final_state=True, use_qk_l2norm_in_kernel=True)
 
-    def micros(beta):
+    def micros(beta, passes=2):
         best = float("inf")
-        for _ in range(2):
+        for _ in range(passes):
             ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
             ev[0].record()
             run(beta)
@@ -625,11 +625,14 @@ def test_chunk_prefill_balanced_segments_bound_their_warm_ups(gdn, dev):
         return best
 
     _, s_ref = run(beta)
-    base, worst = micros(beta), 0.0
+    base, worst = micros(beta, 10), 0.0
     for p in range(T // 64):  # a fast head's warm-up is one chunk: it meets p only from a cut right behind it
         b = beta.clone()
         b[0, 64 * p + 7, h] = 1.5
-        worst = max(worst, micros(b))
+        took = micros(b)
+        if took >= 2 * base:  # (a host that was busy twice in a row)
+            took = min(took, micros(b, 10))
+        worst = max(worst, took)
         if p % 64 == 3:
             _, s = run(b)
             assert rel_l2(s[0, :h], s_ref[0, :h]) <= STATE_TOL
